@@ -275,6 +275,7 @@ struct hpxfft_plan_s
     double row_ms[2] = {};   // measure effort: row pass ms of each kind
     // column strategy
     bool four_step = false;
+    bool col_long = false;   // columns of 2^11 and 2^12 points in one launch (col_long_kernel) instead of the four-step
     int lgP = 0, lgQ = 0;
     int W = 8;
     size_t CW = 0;   // chunk width (columns) of the four-step scratch
@@ -329,6 +330,7 @@ struct hpxfft_plan_s
     int bblocks[2][hpxfft_host::BATCH_NCFG] = {};
     double btune_ms[2][hpxfft_host::BATCH_NCFG] = {};
     double split_ms[COL_TILE_MAX_LG + 1] = {};   // four-step: column-pass ms per tried log2 P (effort >= measure)
+    double long_ms = 0.0;                        // the same of the one-launch form, where it covers the columns
     unsigned *bticket = nullptr;                            // work-queue counters: BATCH_QUEUES per phase
     void *bstage = nullptr;                                 // pinned staging of the grid descriptors, two slots
     hipEvent_t bstage_ev[2] = {nullptr, nullptr};           // each slot's last upload (the slot is free once it ran)
@@ -840,6 +842,13 @@ std::string describe(const hpxfft_plan_s *p)
     else
     {
         const geom ga = tile_geom(p->prec, p->lgQ), gb = tile_geom(p->prec, p->lgP);
+        if (p->col_long)
+        {
+            const int nt = col_long_threads(p->prec, p->lgx, p->ncols, p->batch);
+            os << "  column c2c kernel: " << p->nx << "-point, " << col_long_width(p->prec, p->lgx, nt)
+               << " adjacent columns x all rows in registers, " << nt << " threads, radix 16, LDS "
+               << "exchange in re/im halves; the four-step it replaces:\n";
+        }
         os << "  column c2c four-step Nx = P*Q = " << (1 << p->lgP) << " * " << (1 << p->lgQ) << " (scratch "
            << p->scratch_bytes << " B, one block per strip)\n";
         os << "    phase A: " << (1 << p->lgQ) << "-point DFTs over rows m1+P*m2, twiddle w_Nx^(m1 k2), tiles of "
@@ -853,6 +862,7 @@ std::string describe(const hpxfft_plan_s *p)
             os << "    split autotuned (column pass ms):";
             for (int l = 0; l <= COL_TILE_MAX_LG; ++l)
                 if (p->split_ms[l] > 0.0) os << " P=" << (1 << l) << ": " << p->split_ms[l];
+            if (p->long_ms > 0.0) os << " one launch: " << p->long_ms;
             os << "\n";
         }
     }
@@ -1309,6 +1319,17 @@ int run_columns(hpxfft_plan_s *p, const void *spec_in, void *spec_out, bool conj
         HIPCHK(hipGetLastError());
         return HPXFFT_OK;
     }
+    if (p->col_long)
+    {
+        a.in = spec_in;
+        a.out = spec_out;
+        a.tw_L = tw_ptr(p, p->nx);
+        a.stw64 = p->tabs.stw64;
+        const int nt = col_long_threads(p->prec, p->lgx, p->ncols, p->batch);
+        HIPCHK(col_long(p->prec, p->lgx, conj, a, cdiv(p->ncols, (size_t)col_long_width(p->prec, p->lgx, nt)),
+                        (unsigned)p->batch, nt, p->stream));
+        return HPXFFT_OK;
+    }
     if (!p->four_step)
     {
         a.in = spec_in;
@@ -1442,7 +1463,7 @@ int exec_forward(hpxfft_plan_s *p, const void *d_in, void *d_out, const int *in_
         return rc;
     if (p->timed) HIPCHK(hipEventRecord(p->ev[2], p->stream));
     p->ran = p->timed;
-    p->col_split = p->four_step;
+    p->col_split = p->four_step && !p->col_long;
     p->col_first = false;
     p->h2d = p->d2h = 0.0;
     return HPXFFT_OK;
@@ -1507,7 +1528,7 @@ int exec_wide16(hpxfft_plan_s *p, const void *d_in, void *d_out, const int *in_e
     HIPCHK(hipGetLastError());
     if (p->timed) HIPCHK(hipEventRecord(p->ev[2], p->stream));
     p->ran = p->timed;
-    p->col_split = w->four_step;
+    p->col_split = w->four_step && !w->col_long;
     p->col_first = false;
     p->h2d = p->d2h = 0.0;
     return HPXFFT_OK;
@@ -1545,10 +1566,17 @@ int tune_split(hpxfft_plan_s *p)
     double best_ms = 0.0;
     hipError_t e = hipMemsetAsync(tmp, 0, bytes, p->stream);
     if (e == hipSuccess && s16) e = hipMemsetAsync(p->mid_exp, 0, sizeof(int) * p->nx * p->batch, p->stream);
-    for (int l = lo; l <= hi && e == hipSuccess && rc == HPXFFT_OK; ++l)
+    const bool covers = col_long_covers(p->prec, p->lgx);
+    bool best_long = false;
+    // l = hi + 1: the one-launch form, where it covers the columns
+    for (int l = lo; l <= hi + (covers ? 1 : 0) && e == hipSuccess && rc == HPXFFT_OK; ++l)
     {
-        p->lgP = l;
-        p->lgQ = p->lgx - l;
+        p->col_long = l > hi;
+        if (!p->col_long)
+        {
+            p->lgP = l;
+            p->lgQ = p->lgx - l;
+        }
         const int REPS = tune_reps(p->effort);
         rc = run_columns(p, tmp, tmp, false, s16 ? p->col_exp_own : nullptr);   // warm-up
         if (rc == HPXFFT_OK) e = hipEventRecord(p->ev[0], p->stream);
@@ -1559,14 +1587,20 @@ int tune_split(hpxfft_plan_s *p)
         if (rc == HPXFFT_OK && e == hipSuccess)
         {
             const double ms = elapsed(p->ev[0], p->ev[2]) * 1e3 / REPS;
-            p->split_ms[l] = ms;
-            if (best_ms == 0.0 || ms < best_ms) { best_ms = ms; best = l; }
+            (p->col_long ? p->long_ms : p->split_ms[l]) = ms;
+            if (best_ms == 0.0 || ms < best_ms)
+            {
+                best_ms = ms;
+                best_long = p->col_long;
+                if (!best_long) best = l;
+            }
         }
     }
     (void)hipStreamSynchronize(p->stream);
     (void)hipFree(tmp);
     p->lgP = best;
     p->lgQ = p->lgx - best;
+    p->col_long = best_long;
     if (rc != HPXFFT_OK) return rc;
     HIPCHK(e);
     return HPXFFT_OK;
@@ -1744,6 +1778,9 @@ int choose_columns(hpxfft_plan_s *p)
     const size_t tw_cols = (size_t)tile_geom(p->prec, p->lgQ).nseq;
     p->CW = (p->ncols + tw_cols - 1) / tw_cols * tw_cols;
     p->scratch_bytes = p->nx * p->CW * cb * p->batch;
+    // 2^11 and 2^12 rows, FP64 / FP32: one launch (fft_col_long.hpp), measured
+    // faster at every width; the split stays for hpxfft_plan_set_column_split
+    p->col_long = col_long_covers(p->prec, p->lgx);
     return HPXFFT_OK;
 }
 
@@ -2364,7 +2401,7 @@ int exec_backward(hpxfft_plan_s *plan, const void *d_spec, void *d_real, bool ha
     }
     HIPCHK(hipEventRecord(plan->ev[2], plan->stream));
     plan->ran = true;
-    plan->col_split = plan->four_step;
+    plan->col_split = plan->four_step && !plan->col_long;
     plan->col_first = true;
     return HPXFFT_OK;
 }
@@ -2722,6 +2759,7 @@ int hpxfft_plan_set_column_split(hpxfft_plan plan, int log2_p)
                                             std::to_string(hi) + "] for Nx = " + std::to_string(plan->nx));
     // the scratch holds TW-column strips of Nx rows whatever the split, and the
     // 16-bit column maxima were sized for the largest P of the range
+    plan->col_long = false;
     plan->lgP = log2_p;
     plan->lgQ = plan->lgx - log2_p;
     return HPXFFT_OK;

@@ -1,0 +1,153 @@
+// fft_col_long.hpp -- columns of 2^11 and 2^12 points (FP64 / FP32 storage)
+// in one launch: a workgroup of NT threads holds W adjacent columns over all
+// Nx rows in VGPRs, so the spectrum crosses HBM once in each direction instead
+// of twice through the four-step's scratch.
+//
+// What bounds it: HBM, at the rate of its row segments, plus the transform
+// itself (one or two workgroups share a CU, so little of it is hidden).  512
+// threads hold 2^13 FP64 or 2^14 FP32 points (64 VGPRs of data each), two
+// workgroups per CU: 64-byte segments at 2^11 rows, 32 bytes at 2^12; 1024
+// threads hold twice that, one per CU: 64 bytes at 2^12.  Moving 2 GiB in place
+// in 64-byte segments with no arithmetic runs at 4.3 TB/s of read + write (32
+// bytes 3.2, 16 bytes 1.9), against the four-step's two launches at 5.2, 2.6 per
+// byte of spectrum.  Column pass, four-step -> one launch (us): FP64 2^11 rows x
+// 512, 2048, 8192 reals 20.8 -> 14.7, 32.2 -> 24.1, 109 -> 63, 16 x 2048^2
+// 461 -> 287; FP64 4096^2 115 -> 83, 4 x 4096^2 458 -> 384; FP32 16 x 2048^2
+// 221 -> 160, 16 x 4096^2 857 -> 750.  At 2^13 rows (32-byte segments, 1024
+// threads) it was even with the four-step (8192^2 FP64 465 against 478, FP32
+// slower), so those columns keep the four-step.
+//
+// Radix-16 Stockham stages with one LDS exchange each, then (2^11) a last stage
+// of radix 8.  LDS rows are [pad(e)][w], real and imaginary halves exchanged
+// separately.  Stage twiddles come from the radix-16 stage tables of the long
+// rows (fft_row_big.hpp).
+#pragma once
+
+#include "fft_row_big.hpp"
+
+namespace hpxfft_dev {
+
+constexpr int COL_LONG_MIN_LG = 11, COL_LONG_MAX_LG = 12;
+
+template <typename T, int LG, int NTH> struct collong
+{
+    static constexpr int L = 1 << LG;
+    static constexpr int NB = 8 / (int)sizeof(T);               // radix-16 butterflies per thread and stage
+    static constexpr int NT = NTH;                               // threads
+    static constexpr int W = NT * 16 * NB / L;          // adjacent columns
+    static constexpr int M = L / 16;                             // butterflies per column
+    static constexpr int JT = NT / W;                   // threads per column
+    static constexpr int NR16 = LG / 4;
+    static constexpr int RL = 1 << (LG % 4);                     // last radix (1: none)
+    static constexpr int NSL = L / RL;
+    static constexpr int LP = L + L / 16;
+    static constexpr int ns(int s) { return s == 0 ? 1 : 16 * ns(s - 1); }
+    __device__ static __forceinline__ int pad(int e) { return e + (e >> 4); }
+    static_assert(W >= 1 && JT * NB == M, "threads cover the butterflies");
+};
+
+// exchange: this thread's outputs of radix-16 stage S to LDS, then the inputs of
+// the next stage of radix R2 (element j + r L/R2 of butterfly j = jj + i JT)
+template <typename T, int LG, int NTH, int S, int R2>
+__device__ __forceinline__ void col_long_exchange(cpx<T> *v, T *lds, int jj, int w)
+{
+    using C = collong<T, LG, NTH>;
+    constexpr int NS = C::ns(S), WS = NS == 1 ? 1 : NS + NS / 16, STR = C::L / R2, RS = STR + STR / 16;
+    int wb[C::NB];
+#pragma unroll
+    for (int b = 0; b < C::NB; ++b)
+    {
+        const int j = jj + b * C::JT, k = j & (NS - 1);
+        wb[b] = C::pad((j / NS) * 16 * NS + k) * C::W + w;
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+    {
+#pragma unroll
+        for (int b = 0; b < C::NB; ++b)
+#pragma unroll
+            for (int q = 0; q < 16; ++q) lds[wb[b] + q * WS * C::W] = h ? v[16 * b + q].y : v[16 * b + q].x;
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 16 * C::NB / R2; ++i)
+        {
+            const int rb = C::pad(jj + i * C::JT) * C::W + w;
+#pragma unroll
+            for (int r = 0; r < R2; ++r)
+            {
+                if (h) v[i * R2 + r].y = lds[rb + r * RS * C::W];
+                else v[i * R2 + r].x = lds[rb + r * RS * C::W];
+            }
+        }
+        if (h == 0) __syncthreads();
+    }
+}
+
+template <typename T, int LG, int NTH, int S>
+__device__ __forceinline__ void col_long_stages(cpx<T> *v, T *lds, const cpx<double> *__restrict__ stw64, int jj, int w)
+{
+    using C = collong<T, LG, NTH>;
+    constexpr int NS = C::ns(S);
+#pragma unroll
+    for (int b = 0; b < C::NB; ++b)
+    {
+        if constexpr (NS > 1) twiddle16<T, NS>(v + 16 * b, stw64, (jj + b * C::JT) & (NS - 1));
+        dft16(v + 16 * b);
+    }
+    if constexpr (S + 1 < C::NR16)
+    {
+        if constexpr (S > 0) __syncthreads();   // the last exchange's reads
+        col_long_exchange<T, LG, NTH, S, 16>(v, lds, jj, w);
+        col_long_stages<T, LG, NTH, S + 1>(v, lds, stw64, jj, w);
+    }
+}
+
+// blockIdx.x = strip, .z = grid; from a.in to a.out in the same layout (in
+// place for the forward transform).  CONJ: the inverse, conj(DFT(conj .)).
+template <typename T, int LG, int NTH, bool CONJ>
+__global__ void __launch_bounds__(NTH, 4) col_long_kernel(ColArgs a)
+{
+    using C = collong<T, LG, NTH>;
+    constexpr int W = C::W, JT = C::JT, M = C::M, RL = C::RL, NSL = C::NSL, NB = C::NB;
+    __shared__ T lds[C::LP * W];
+    const int t = threadIdx.x, w = t % W, jj = t / W;
+    const blk3 bk = xcd_block();   // neighbouring strips share lines: one XCD
+    const int c = bk.x * W + w;
+    const bool valid = c < a.ncols;
+    const int cl = valid ? c : a.ncols - 1;   // lanes past the last column load it and store nothing
+    const long long base = (long long)bk.z * a.dist + cl + (long long)jj * a.pitch;
+    const T *in = reinterpret_cast<const T *>(a.in) + 2 * base;
+    T *out = reinterpret_cast<T *>(a.out) + 2 * base;
+    cpx<T> v[16 * NB];
+#pragma unroll
+    for (int u = 0; u < 16 * NB; ++u)
+    {
+        cpx<T> z = stor<T>::ld(in + 2 * a.pitch * ((u / 16) * JT + (u % 16) * M));
+        v[u] = CONJ ? conjc(z) : z;
+    }
+    col_long_stages<T, LG, NTH, 0>(v, lds, reinterpret_cast<const cpx<double> *>(a.stw64), jj, w);
+    if constexpr (RL > 1)
+    {
+        // last stage: butterfly j reads j + r NSL, outputs j + q NSL; twiddles w_L^{r j}
+        __syncthreads();
+        col_long_exchange<T, LG, NTH, C::NR16 - 1, RL>(v, lds, jj, w);
+        const cpx<T> *tw = reinterpret_cast<const cpx<T> *>(a.tw_L);
+#pragma unroll
+        for (int i = 0; i < 16 * NB / RL; ++i)
+        {
+#pragma unroll
+            for (int r = 1; r < RL; ++r) v[i * RL + r] = cmul(v[i * RL + r], tw[r * (jj + i * JT)]);
+            dftR<T, RL>(v + i * RL);
+        }
+    }
+    if (!valid) return;
+    constexpr int R = RL > 1 ? RL : 16, STR = RL > 1 ? NSL : M;
+#pragma unroll
+    for (int u = 0; u < 16 * NB; ++u)
+    {
+        const cpx<T> z = v[u];
+        stor<T>::st(out + 2 * a.pitch * ((u / R) * JT + (u % R) * STR), CONJ ? conjc(z) : z);
+    }
+}
+
+}   // namespace hpxfft_dev

@@ -88,6 +88,7 @@ struct ColArgs
     const void *tw_N;  // w_Nx^m, m < Nx (MODE 1 post-twiddle)
     const void *tw64_L;  // the same tables in FP64 (FP32 four-step tiles form their twiddles in FP64)
     const void *tw64_N;
+    const void *stw64;   // radix-16 stage twiddles of the one-launch long columns (stage_tw_off), FP64
     const int *row_exp;    // 16-bit inputs (MODE 0,1): per-row exponent of the rows
     unsigned *colpart;     // 16-bit four-step phase A: per-workgroup column maxima [m1][ncols] (float bits)
     unsigned *colmax;      // 16-bit four-step phase B: per-column maxima (reduced from colpart)

@@ -3,3 +3,4 @@
 #include "launch.hpp"
 
 HPXFFT_DEFINE_LAUNCH(f32, float, float, true)
+HPXFFT_DEFINE_COL_LONG(f32, float)

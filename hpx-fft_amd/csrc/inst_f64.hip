@@ -3,3 +3,4 @@
 #include "launch.hpp"
 
 HPXFFT_DEFINE_LAUNCH(f64, double, double, true)
+HPXFFT_DEFINE_COL_LONG(f64, double)

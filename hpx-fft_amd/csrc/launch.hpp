@@ -5,6 +5,7 @@
 #include "fft_row_big.hpp"
 #include "fft_row_pair.hpp"
 #include "fft_tile.hpp"
+#include "fft_col_long.hpp"
 #include <algorithm>
 
 namespace hpxfft_host {
@@ -42,6 +43,40 @@ HPXFFT_DECL_LAUNCH(f64)
 HPXFFT_DECL_LAUNCH(f32)
 HPXFFT_DECL_LAUNCH(f16)
 HPXFFT_DECL_LAUNCH(bf16)
+
+// columns of 2^11 and 2^12 points in one launch (fft_col_long.hpp; FP64 / FP32):
+// gx strips of col_long_width columns, gz grids, nt threads per workgroup
+hipError_t col_long_f64(int lg, bool conj, const ColArgs &a, unsigned gx, unsigned gz, int nt, hipStream_t s);
+hipError_t col_long_f32(int lg, bool conj, const ColArgs &a, unsigned gx, unsigned gz, int nt, hipStream_t s);
+inline hipError_t col_long(int p, int lg, bool conj, const ColArgs &a, unsigned gx, unsigned gz, int nt, hipStream_t s)
+{
+    switch (p)
+    {
+    case P_F64: return col_long_f64(lg, conj, a, gx, gz, nt, s);
+    case P_F32: return col_long_f32(lg, conj, a, gx, gz, nt, s);
+    default: return hipErrorInvalidValue;
+    }
+}
+inline bool col_long_covers(int prec, int lg)
+{
+    return (prec == P_F64 || prec == P_F32) && lg >= hpxfft_dev::COL_LONG_MIN_LG && lg <= hpxfft_dev::COL_LONG_MAX_LG;
+}
+// adjacent columns per workgroup of nt threads (64 VGPRs of data per thread)
+inline int col_long_width(int prec, int lg, int nt) { return (nt * (prec == P_F64 ? 16 : 32)) >> lg; }
+// threads per workgroup.  2^11 rows: 512 (64-byte row segments, two workgroups
+// per CU; 1024 threads with 128-byte segments were slower up to 4096 reals per
+// row and even beyond).  2^12 rows: 1024 (64-byte segments, one workgroup per
+// CU), except where that leaves CUs idle and the narrow form's twice as many
+// workgroups win: a launch of less than about a third of the 256 CUs (FP64 4096
+// x 512, 65 strips: 23.2 -> 19.5 us; 4096 x 1024, 129 strips: 25.2 against
+// 27.9), or one whose second round would hold a few strips (4096 x 2048, 257
+// strips: 46.3 -> 41.2)
+inline int col_long_threads(int prec, int lg, size_t ncols, size_t batch)
+{
+    if (lg == 11) return 512;
+    const size_t w = (size_t)col_long_width(prec, lg, 1024), strips = (ncols + w - 1) / w * batch;
+    return strips <= 96 || (strips > 256 && strips <= 288) ? 512 : 1024;
+}
 
 // rows of 2^13 / 2^14 complex points with lane-pair radix-32 stages
 // (fft_row_pair.hpp; FP32 arithmetic: FP32 and 16-bit storage); `total` rows
@@ -203,6 +238,22 @@ hipError_t launch_col(const ColArgs &a, unsigned gx, unsigned gy, unsigned gz, h
     return hipGetLastError();
 }
 
+template <typename T, int LG, int NT>
+void launch_col_long_nt(bool conj, const ColArgs &a, unsigned gx, unsigned gz, hipStream_t s)
+{
+    if (conj) hipLaunchKernelGGL((col_long_kernel<T, LG, NT, true>), dim3(gx, 1, gz), dim3(NT), 0, s, a);
+    else hipLaunchKernelGGL((col_long_kernel<T, LG, NT, false>), dim3(gx, 1, gz), dim3(NT), 0, s, a);
+}
+template <typename T>
+hipError_t launch_col_long(int lg, bool conj, const ColArgs &a, unsigned gx, unsigned gz, int nt, hipStream_t s)
+{
+    if (lg == 11 && nt == 512) launch_col_long_nt<T, 11, 512>(conj, a, gx, gz, s);
+    else if (lg == 12 && nt == 512) launch_col_long_nt<T, 12, 512>(conj, a, gx, gz, s);
+    else if (lg == 12 && nt == 1024) launch_col_long_nt<T, 12, 1024>(conj, a, gx, gz, s);
+    else return hipErrorInvalidValue;
+    return hipGetLastError();
+}
+
 template <typename T, typename S, int LG = 0>
 hipError_t row_r2c_sw(int lg, const RowArgs &a, unsigned gx, unsigned gy, hipStream_t s)
 {
@@ -280,6 +331,14 @@ template <typename T, typename S> geom tile_geom_t(int lg)
 }   // namespace detail
 }   // namespace hpxfft_host
 
+#define HPXFFT_DEFINE_COL_LONG(sfx, T)                                                                             \
+    namespace hpxfft_host {                                                                                        \
+    hipError_t col_long_##sfx(int lg, bool conj, const ColArgs &a, unsigned gx, unsigned gz, int nt,               \
+                              hipStream_t s)                                                                       \
+    {                                                                                                              \
+        return detail::launch_col_long<T>(lg, conj, a, gx, gz, nt, s);                                             \
+    }                                                                                                              \
+    }
 #define HPXFFT_DEFINE_LAUNCH(sfx, T, S, ADJ)                                                                         \
     namespace hpxfft_host {                                                                                        \
     hipError_t row_r2c_##sfx(int lg, const RowArgs &a, unsigned gx, unsigned gy, hipStream_t s)                    \

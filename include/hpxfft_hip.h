@@ -65,8 +65,9 @@ typedef enum
  * as FFTW_MEASURE < FFTW_PATIENT < FFTW_EXHAUSTIVE, adapter_fftw.hpp:13-18). */
 typedef enum
 {
-    HPXFFT_ESTIMATE = 0,   /* no timing: balanced four-step split, radix-16 row kernel, in-place general stages */
-    HPXFFT_MEASURE = 1,    /* time the four-step splits, the general kernels' stage forms and one/two levels,
+    HPXFFT_ESTIMATE = 0,   /* no timing: one-launch columns up to 2^12 rows (FP64 / FP32), else the balanced
+                              four-step split; radix-16 row kernel, in-place general stages */
+    HPXFFT_MEASURE = 1,    /* time the four-step splits (and the one-launch form), the general kernels' stage forms and one/two levels,
                               the batched task shapes; keep the fastest (3 timed runs per candidate) */
     HPXFFT_PATIENT = 2,    /* measure's search, plus the row kernels of 2^13- / 2^14-point rows (FP32
                               arithmetic); 5 timed runs per candidate */
@@ -112,9 +113,9 @@ int hpxfft_exec_r2c_2d(hpxfft_plan plan, const void *d_in, void *d_out);
  * planned as hpxfft_plan_r2c_2d at "estimate" on every call and enqueued on
  * `stream` (a hipStream_t, NULL = default) with no plan object: the results
  * equal that plan's bit for bit.  No hipMalloc, hipFree or other allocation
- * happens.  A column pass that runs as a four-step (Nx > 1024) keeps its
+ * happens.  A column pass that runs as a four-step (Nx > 4096) keeps its
  * intermediate in a static device array of 128 MiB (134217728 bytes) per
- * device, held until the process ends; a grid whose intermediate,
+ * device, held until the process ends; a grid with Nx > 1024 whose intermediate,
  * Nx x (Ny/2+1) complex values of the precision (rounded up to whole strips
  * of 32 FP64 or 64 FP32 columns), exceeds it is refused with
  * HPXFFT_UNSUPPORTED_SIZE.  Every call on a device shares that device's array:
@@ -167,8 +168,9 @@ int hpxfft_exec_c2r_2d(hpxfft_plan plan, const void *d_spec, void *d_real);
  * the last exec for "total", "first_fftw", "first_trans", "second_fftw",
  * "second_trans" (the transposes are fused into the column pass and read
  * 0), "h2d", "d2h"; "plan" (planning seconds) and "plan_flops"; and, when
- * the column pass runs as two launches (Nx > 1024, or > 512 for 16-bit
- * storage), "column_a" and "column_b" (seconds of each launch of the last
+ * the column pass runs as two launches (a four-step: Nx > 4096, or > 512 for
+ * 16-bit storage, or a split set by the caller or chosen by the measure
+ * effort), "column_a" and "column_b" (seconds of each launch of the last
  * exec; 0 otherwise).  The backward execs (adjoint, c2r) run the column
  * pass first: for them "first_fftw" is the column pass and "second_fftw"
  * the row pass; batched plans give their row and column launches.  Unknown keys
@@ -213,12 +215,13 @@ int hpxfft_plan_batched_set_config(hpxfft_plan plan, int row_cfg, int col_cfg);
 
 /* No reference counterpart (FFTW's planner choice is internal to
  * fftw_plan_dft_1d, core/src/util/adapter_fftw.cpp:28-29): runs the plan's
- * four-step column pass with the split Nx = P * Q, P = 2^log2_p, instead of
- * the one it chose (estimate: the balanced split; measure and above: the
- * fastest one timed).  log2_p must lie in the range of splits the kernels
- * cover (sub-lengths 2^5 .. 2^8).  HPXFFT_INVALID_ARG for another value or
- * for a plan whose column pass is not a four-step (the plan text says which
- * it is).  Lets a test check every split the measure effort may keep. */
+ * column pass as the four-step with the split Nx = P * Q, P = 2^log2_p, instead
+ * of what it chose (estimate: one launch up to 2^12 rows in FP64 / FP32, the
+ * balanced split beyond; measure and above: the fastest one timed).  log2_p
+ * must lie in the range of splits the kernels cover (sub-lengths 2^5 .. 2^8).
+ * HPXFFT_INVALID_ARG for another value or for a plan whose columns have no
+ * four-step (the plan text lists it where there is one).  Lets a test check
+ * every split the measure effort may keep. */
 int hpxfft_plan_set_column_split(hpxfft_plan plan, int log2_p);
 
 /* No reference counterpart: selects the row kernel of a plan whose rows are
