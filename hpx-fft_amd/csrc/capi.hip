@@ -311,11 +311,17 @@ struct hpxfft_plan_s
     void *host_buf = nullptr;     // drop-in host path: device copy of the vector_2d
     size_t host_bytes = 0;
     // timing
-    hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};   // start, rows done, columns done, column phase A done
+    hipEvent_t ev[2] = {nullptr, nullptr};   // of the planning searches
+    // device words the kernels stamp with the wall clock (Stamps): [ST_START]
+    // the first launch's start, [ST_MID] the second pass's, [ST_SPLIT] the
+    // four-step phase B's, then STAMP_SLOTS ends of the last launch's workgroups
+    unsigned long long *stamps = nullptr;   // null: untimed (the allocation-free entry point)
+    int stamp_set = -1;          // index in the device's pool of sets (alloc_timing); -1: an allocation
+    bool own_ends = true;        // false: the exec is the middle of a longer one, which stamps start and end itself
+    double clock_hz = 1e8;
     bool ran = false;
-    bool timed = true;           // exec records the phase events (off for the allocation-free entry point)
-    bool col_split = false;      // ev[3] valid: the last run's column pass was a four-step
-    bool col_first = false;      // the last run was backward: column pass (ev0..ev1) before the rows
+    bool col_split = false;      // the last run's column pass was a four-step
+    bool col_first = false;      // the last run was backward: the column pass before the rows
     double h2d = 0.0, d2h = 0.0;
     double plan_seconds = 0.0, plan_flops = 0.0;
     std::map<std::string, double> extra;
@@ -339,6 +345,11 @@ struct hpxfft_plan_s
 };
 
 namespace {
+
+enum { ST_START = 0, ST_MID = 1, ST_SPLIT = 2, ST_END = 8, ST_WORDS = ST_END + hpxfft_dev::STAMP_SLOTS };
+unsigned long long *stamp_at(const hpxfft_plan_s *p, int i) { return p->stamps ? p->stamps + i : nullptr; }
+unsigned long long *stamp_start(const hpxfft_plan_s *p) { return p->own_ends ? stamp_at(p, ST_START) : nullptr; }
+unsigned long long *stamp_ends(const hpxfft_plan_s *p) { return p->own_ends ? stamp_at(p, ST_END) : nullptr; }
 
 const void *tw_ptr(const hpxfft_plan_s *p, size_t N)
 {
@@ -894,10 +905,74 @@ double elapsed(hipEvent_t a, hipEvent_t b)
     return (double)ms * 1e-3;
 }
 
+// Stamp words for the plans of a device: STAMP_POOL sets in a static array (one
+// copy per device, zero from the start), handed out under a lock and given back
+// by free_plan; a further plan allocates its own.  A set's old values need no
+// clearing: the start words are rewritten by every exec, and earlier ends never
+// exceed later ones.  (hipMalloc and a clearing copy took 30 us per plan.)
+constexpr int STAMP_POOL = 64;
+static __device__ unsigned long long stamp_pool[STAMP_POOL][ST_WORDS];
+std::mutex g_stamp_mu;
+struct stamp_sets { unsigned long long *base = nullptr; uint64_t used = 0; };
+std::map<int, stamp_sets> g_stamps;
+
+// a set of stamp words for a new plan on its device (current)
+int alloc_timing(hpxfft_plan_s *p)
+{
+    int khz = 0;
+    HIPCHK(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, p->device));
+    if (khz > 0) p->clock_hz = 1e3 * khz;
+    {
+        std::lock_guard<std::mutex> lk(g_stamp_mu);
+        stamp_sets &d = g_stamps[p->device];
+        if (!d.base) HIPCHK(hipGetSymbolAddress(reinterpret_cast<void **>(&d.base), HIP_SYMBOL(stamp_pool)));
+        for (int i = 0; i < STAMP_POOL; ++i)
+            if (!(d.used >> i & 1))
+            {
+                d.used |= uint64_t(1) << i;
+                p->stamp_set = i;
+                p->stamps = d.base + (size_t)i * ST_WORDS;
+                return HPXFFT_OK;
+            }
+    }
+    HIPCHK(hipMalloc(&p->stamps, sizeof(unsigned long long) * ST_WORDS));
+    const std::vector<unsigned long long> zero(ST_WORDS, 0);
+    HIPCHK(hipMemcpy(p->stamps, zero.data(), sizeof(zero[0]) * ST_WORDS, hipMemcpyHostToDevice));
+    return HPXFFT_OK;
+}
+void free_timing(hpxfft_plan_s *p)
+{
+    if (p->stamp_set >= 0)
+    {
+        std::lock_guard<std::mutex> lk(g_stamp_mu);
+        g_stamps[p->device].used &= ~(uint64_t(1) << p->stamp_set);
+    }
+    else (void)hipFree(p->stamps);
+}
+
+// the planning searches' events
 int alloc_events(hpxfft_plan_s *p)
 {
     for (auto &e : p->ev)
         if (!e) HIPCHK(hipEventCreate(&e));
+    return HPXFFT_OK;
+}
+
+// seconds of the last exec's phases, once it has finished
+struct phase_times { double total, first, second, split_a, split_b; };
+int read_times(hpxfft_plan_s *p, phase_times &t)
+{
+    std::vector<unsigned long long> w(ST_WORDS);
+    HIPCHK(hipMemcpyAsync(w.data(), p->stamps, sizeof(w[0]) * ST_WORDS, hipMemcpyDeviceToHost, p->stream));
+    HIPCHK(hipStreamSynchronize(p->stream));
+    const unsigned long long end = *std::max_element(w.begin() + ST_END, w.end());
+    auto s = [&](unsigned long long a, unsigned long long b) { return b > a ? (double)(b - a) / p->clock_hz : 0.0; };
+    t.total = s(w[ST_START], end);
+    t.first = s(w[ST_START], w[ST_MID]);
+    t.second = s(w[ST_MID], end);
+    // the split lies in the column pass: second after forward execs, first after backward ones
+    t.split_a = p->col_first ? s(w[ST_START], w[ST_SPLIT]) : s(w[ST_MID], w[ST_SPLIT]);
+    t.split_b = p->col_first ? s(w[ST_SPLIT], w[ST_MID]) : s(w[ST_SPLIT], end);
     return HPXFFT_OK;
 }
 
@@ -959,7 +1034,7 @@ void blue_fields(const hpxfft_plan_s *p, const gen2_dim &d, hpxfft_dev::GenStrid
 
 // two-level Bluestein column pass (Nx = N, M = P*Q) from spec_in to spec_out
 // through the plan's scratch [m1][k2][col] of M rows; conj: the inverse
-int run_columns_blue(hpxfft_plan_s *p, const void *spec_in, void *spec_out, bool conj)
+int run_columns_blue(hpxfft_plan_s *p, const void *spec_in, void *spec_out, bool conj, hpxfft_dev::Stamps ts)
 {
     const gen2_dim &d = p->g2c;
     const long long P = d.P, Q = d.Q, M = (long long)d.points(), nc = (long long)p->ncols, ld = (long long)p->ld_out;
@@ -980,6 +1055,7 @@ int run_columns_blue(hpxfft_plan_s *p, const void *spec_in, void *spec_out, bool
     a.tw_shift = d.tw_shift;
     a.conj_in = conj;
     a.blue_in = 1;
+    a.ts.begin = ts.begin;
     blue_fields(p, d, a);
     if (int rc = launch_strided(p, a, d.A, d.tabA, d.tabT, d.WA, cdiv(nc, d.WA), (unsigned)P, bz)) return rc;
     hpxfft_dev::GenStride m{};
@@ -1006,6 +1082,7 @@ int run_columns_blue(hpxfft_plan_s *p, const void *spec_in, void *spec_out, bool
     b.conj_in = b.conj_out = 1;
     b.blue_out = 1;
     b.blue_conj = conj;
+    b.ts.end = ts.end;
     blue_fields(p, d, b);
     return launch_strided(p, b, d.A, d.tabA, d.tabT, d.WA, cdiv(nc, d.WA), (unsigned)P, bz);
 }
@@ -1015,7 +1092,7 @@ int run_columns_blue(hpxfft_plan_s *p, const void *spec_in, void *spec_out, bool
 // points -> the spectrum rows, then the r2c split in place.  Backward (c2r,
 // halve for the adjoint): the c2r sequence of each half-spectrum row -> `real`.
 int run_rows_blue(hpxfft_plan_s *p, const void *real_in, void *real_out, const void *spec_in, void *spec_out,
-                  bool backward, bool halve)
+                  bool backward, bool halve, hpxfft_dev::Stamps ts)
 {
     const gen2_dim &d = p->g2r;
     const long long P = d.P, Q = d.Q, M = (long long)d.points(), L = (long long)d.N, nx = (long long)p->nx;
@@ -1049,6 +1126,7 @@ int run_rows_blue(hpxfft_plan_s *p, const void *real_in, void *real_out, const v
     a.tw_col = 1;
     a.tw_shift = d.tw_shift;
     a.blue_in = 1;
+    a.ts.begin = ts.begin;
     blue_fields(p, d, a);
     if (int rc = launch_strided(p, a, d.A, d.tabA, d.tabT, d.WA, cdiv(P, d.WA), by, bz)) return rc;
     hpxfft_dev::GenStride m{};
@@ -1073,6 +1151,7 @@ int run_rows_blue(hpxfft_plan_s *p, const void *real_in, void *real_out, const v
     b.tw_col = 1;
     b.conj_in = b.conj_out = 1;
     b.blue_out = 1;
+    b.ts.end = ts.end;
     blue_fields(p, d, b);
     if (!backward)
     {
@@ -1105,9 +1184,9 @@ int run_rows_blue(hpxfft_plan_s *p, const void *real_in, void *real_out, const v
 
 // two-level column pass (Nx = P*Q) from spec_in to spec_out through the
 // plan's scratch [m1][k2][col]; conj: the inverse transform
-int run_columns_2level(hpxfft_plan_s *p, const void *spec_in, void *spec_out, bool conj)
+int run_columns_2level(hpxfft_plan_s *p, const void *spec_in, void *spec_out, bool conj, hpxfft_dev::Stamps ts)
 {
-    if (p->g2c.blue) return run_columns_blue(p, spec_in, spec_out, conj);
+    if (p->g2c.blue) return run_columns_blue(p, spec_in, spec_out, conj, ts);
     const gen2_dim &d = p->g2c;
     const long long P = d.P, Q = d.Q, nc = (long long)p->ncols, ld = (long long)p->ld_out;
     hpxfft_dev::GenStride a{};
@@ -1125,6 +1204,7 @@ int run_columns_2level(hpxfft_plan_s *p, const void *spec_in, void *spec_out, bo
     a.tw_n = (int)p->nx;
     a.tw_shift = d.tw_shift;
     a.conj_in = conj;
+    a.ts.begin = ts.begin;
     if (int rc = launch_strided(p, a, d.A, d.tabA, d.tabT, d.WA, cdiv(nc, d.WA), (unsigned)P, (unsigned)p->batch))
         return rc;
     hpxfft_dev::GenStride b{};
@@ -1140,6 +1220,7 @@ int run_columns_2level(hpxfft_plan_s *p, const void *spec_in, void *spec_out, bo
     b.out_bat = (long long)p->dist_out;
     b.ncols = (int)nc;
     b.conj_out = conj;
+    b.ts.end = ts.end;
     return launch_strided(p, b, d.B, d.tabB, d.tabT, d.WB, cdiv(nc, d.WB), (unsigned)Q, (unsigned)p->batch);
 }
 
@@ -1162,9 +1243,9 @@ int rows_split_width(const hpxfft_plan_s *p, hpxfft_dev::GenPlan &gB)
 // r2c split in place.  Backward (c2r, halve for the adjoint): the c2r
 // sequence of each half-spectrum row of `spec` -> scratch -> `real`.
 int run_rows_2level(hpxfft_plan_s *p, const void *real_in, void *real_out, const void *spec_in, void *spec_out,
-                    bool backward, bool halve)
+                     bool backward, bool halve, hpxfft_dev::Stamps ts)
 {
-    if (p->g2r.blue) return run_rows_blue(p, real_in, real_out, spec_in, spec_out, backward, halve);
+    if (p->g2r.blue) return run_rows_blue(p, real_in, real_out, spec_in, spec_out, backward, halve, ts);
     const gen2_dim &d = p->g2r;
     const long long P = d.P, Q = d.Q, L = P * Q;
     hpxfft_dev::GenStride a{};
@@ -1195,6 +1276,7 @@ int run_rows_2level(hpxfft_plan_s *p, const void *real_in, void *real_out, const
     a.tw_n = (int)L;
     a.tw_col = 1;
     a.tw_shift = d.tw_shift;
+    a.ts.begin = ts.begin;
     if (int rc = launch_strided(p, a, d.A, d.tabA, d.tabT, d.WA, cdiv(P, d.WA), (unsigned)p->nx, (unsigned)p->batch))
         return rc;
     hpxfft_dev::GenPlan gB;
@@ -1251,6 +1333,7 @@ int run_rows_2level(hpxfft_plan_s *p, const void *real_in, void *real_out, const
         b.out_sub = (long long)p->ld_in / 2;
         b.out_bat = (long long)p->dist_in / 2;
         b.conj_out = 1;
+        b.ts.end = ts.end;
     }
     if (int rc = launch_strided(p, b, d.B, d.tabB, d.tabT, d.WB, cdiv(Q, d.WB), (unsigned)p->nx, (unsigned)p->batch))
         return rc;
@@ -1271,8 +1354,10 @@ int run_rows_2level(hpxfft_plan_s *p, const void *real_in, void *real_out, const
 
 // column pass on the spectrum `spec` (in place), or from `spec_in` to
 // `spec_out` for the adjoint; `conj` = inverse transform.
+// ts: stamps of the pass (begin: its first launch, end: its last), split:
+// that of the four-step's second launch.
 int run_columns(hpxfft_plan_s *p, const void *spec_in, void *spec_out, bool conj, int *col_exp,
-                hipEvent_t mid = nullptr)
+                hpxfft_dev::Stamps ts = {nullptr, nullptr}, unsigned long long *split = nullptr)
 {
     const size_t sb = storage_bytes(p->prec);
     const int W = p->four_step ? tile_geom(p->prec, p->lgQ).nseq : p->W;
@@ -1284,7 +1369,8 @@ int run_columns(hpxfft_plan_s *p, const void *spec_in, void *spec_out, bool conj
     a.out_exp = col_exp;
     a.rexp_dist = (long long)p->nx;
     a.cexp_dist = (long long)p->ncols;
-    if (p->g2c.on) return run_columns_2level(p, spec_in, spec_out, conj);
+    a.ts = ts;
+    if (p->g2c.on) return run_columns_2level(p, spec_in, spec_out, conj, ts);
     if (p->gen_col)
     {
         // general length (F64 / F32; in place for the forward transform)
@@ -1356,6 +1442,7 @@ int run_columns(hpxfft_plan_s *p, const void *spec_in, void *spec_out, bool conj
     a.out = p->scratch;
     a.tw_L = tw_ptr(p, (size_t)Q);
     a.tw64_L = tw64_ptr(p, (size_t)Q);
+    a.ts.end = nullptr;
     HIPCHK(col(p->prec, p->lgQ, 1, conj, a, gx, (unsigned)P, nb, p->stream));
     if (p->colpart)
     {
@@ -1364,7 +1451,7 @@ int run_columns(hpxfft_plan_s *p, const void *spec_in, void *spec_out, bool conj
                            0, p->stream, p->colpart, p->colmax, (int)p->ncols, P);
         HIPCHK(hipGetLastError());
     }
-    if (mid) HIPCHK(hipEventRecord(mid, p->stream));
+    a.ts = {split, ts.end};
     // phase B: scratch -> spectrum; its tiles are shifted to whole 128-byte
     // lines of the output rows, which can take one more tile per row
     const int eline = (int)(128 / (2 * sb));
@@ -1412,12 +1499,8 @@ int exec_forward(hpxfft_plan_s *p, const void *d_in, void *d_out, const int *in_
     if (s16 && !col_exp) col_exp = p->col_exp_own;
     if (p->wide16) return exec_wide16(p, d_in, d_out, in_exp, col_exp);
     device_guard g(p->device);
-    if (p->timed)
-    {
-        if (int rc = alloc_events(p)) return rc;
-        HIPCHK(hipEventRecord(p->ev[0], p->stream));
-    }
     RowArgs r{};
+    r.ts.begin = stamp_start(p);
     r.in = d_in;
     r.out = d_out;
     r.ld_in = (long long)p->ld_in;
@@ -1434,7 +1517,7 @@ int exec_forward(hpxfft_plan_s *p, const void *d_in, void *d_out, const int *in_
     r.exp_dist = (long long)p->nx;
     if (p->g2r.on)
     {
-        if (int rc = run_rows_2level(p, d_in, nullptr, nullptr, d_out, false, false)) return rc;
+        if (int rc = run_rows_2level(p, d_in, nullptr, nullptr, d_out, false, false, r.ts)) return rc;
     }
     else if (p->gen_row)
     {
@@ -1458,11 +1541,10 @@ int exec_forward(hpxfft_plan_s *p, const void *d_in, void *d_out, const int *in_
     {
         HIPCHK(launch_rows_pow2(p, r, p->row_kind));
     }
-    if (p->timed) HIPCHK(hipEventRecord(p->ev[1], p->stream));
-    if (int rc = run_columns(p, d_out, d_out, false, s16 ? col_exp : nullptr, p->timed ? p->ev[3] : nullptr))
+    if (int rc = run_columns(p, d_out, d_out, false, s16 ? col_exp : nullptr, {stamp_at(p, ST_MID), stamp_ends(p)},
+                             stamp_at(p, ST_SPLIT)))
         return rc;
-    if (p->timed) HIPCHK(hipEventRecord(p->ev[2], p->stream));
-    p->ran = p->timed;
+    p->ran = p->stamps != nullptr;
     p->col_split = p->four_step && !p->col_long;
     p->col_first = false;
     p->h2d = p->d2h = 0.0;
@@ -1471,8 +1553,8 @@ int exec_forward(hpxfft_plan_s *p, const void *d_in, void *d_out, const int *in_
 
 // 16-bit storage through the FP32 workspace: convert in (unscaling rows by
 // in_exp), the FP32 plan in place, the column maxima, convert out (scaling
-// columns, exponents to col_exp).  Timing: the FP32 plan records the row /
-// column boundaries into this plan's events, so first_fftw covers the
+// columns, exponents to col_exp).  Timing: the FP32 plan's launches stamp the
+// row / column boundaries into this plan's words, so first_fftw covers the
 // conversion in and the rows, second_fftw the columns and the conversion out.
 int exec_wide16(hpxfft_plan_s *p, const void *d_in, void *d_out, const int *in_exp, int *col_exp)
 {
@@ -1480,36 +1562,23 @@ int exec_wide16(hpxfft_plan_s *p, const void *d_in, void *d_out, const int *in_e
     const long long nc = (long long)p->ncols, ldw = 2 * nc, distw = (long long)p->nx * ldw;
     const dim3 gin(cdiv(p->ny / 2, 256), (unsigned)p->nx, (unsigned)p->batch);
     const dim3 gcol(cdiv(p->ncols, 256), (unsigned)p->nx, (unsigned)p->batch);
-    if (p->timed)
-    {
-        if (int rc = alloc_events(p)) return rc;
-        HIPCHK(hipEventRecord(p->ev[0], p->stream));
-    }
     using namespace hpxfft_dev;
+    const Stamps tin = {stamp_start(p), nullptr}, tout = {nullptr, stamp_ends(p)};
     if (p->prec == P_F16)
         hipLaunchKernelGGL(wide_in_kernel<__half>, gin, dim3(256), 0, p->stream, static_cast<const __half *>(d_in),
                            (long long)p->ld_in, (long long)p->dist_in, in_exp, (long long)p->nx, p->wide_ws, ldw,
-                           distw, (int)(p->ny / 2));
+                           distw, (int)(p->ny / 2), tin);
     else
         hipLaunchKernelGGL(wide_in_kernel<bf16_t>, gin, dim3(256), 0, p->stream, static_cast<const bf16_t *>(d_in),
                            (long long)p->ld_in, (long long)p->dist_in, in_exp, (long long)p->nx, p->wide_ws, ldw,
-                           distw, (int)(p->ny / 2));
+                           distw, (int)(p->ny / 2), tin);
     HIPCHK(hipGetLastError());
-    // the FP32 plan records its phase boundaries into this plan's events
-    hipEvent_t own[3] = {w->ev[1], w->ev[2], w->ev[3]};
-    const bool wt = w->timed;
-    if (p->timed)
-    {
-        w->ev[1] = p->ev[1];
-        w->ev[2] = p->ev[2];
-        w->ev[3] = p->ev[3];
-    }
-    w->timed = p->timed;
+    unsigned long long *own = w->stamps;
+    w->stamps = p->stamps;
+    w->own_ends = false;
     const int rc = exec_forward(w, p->wide_ws, p->wide_ws, nullptr, nullptr);
-    w->ev[1] = own[0];
-    w->ev[2] = own[1];
-    w->ev[3] = own[2];
-    w->timed = wt;
+    w->stamps = own;
+    w->own_ends = true;
     if (rc) return rc;
     const long long ncm = (long long)p->ncols * (long long)p->batch;
     hipLaunchKernelGGL(zero_u32_kernel<0>, dim3(cdiv((size_t)ncm, 256)), dim3(256), 0, p->stream, p->colmax, ncm);
@@ -1520,14 +1589,13 @@ int exec_wide16(hpxfft_plan_s *p, const void *d_in, void *d_out, const int *in_e
     if (p->prec == P_F16)
         hipLaunchKernelGGL(wide_out_kernel<__half>, gcol, dim3(256), 0, p->stream, p->wide_ws, ldw, distw,
                            static_cast<__half *>(d_out), (long long)(2 * p->ld_out), (long long)(2 * p->dist_out),
-                           (int)p->ncols, p->colmax, col_exp, (long long)p->ncols);
+                           (int)p->ncols, p->colmax, col_exp, (long long)p->ncols, tout);
     else
         hipLaunchKernelGGL(wide_out_kernel<bf16_t>, gcol, dim3(256), 0, p->stream, p->wide_ws, ldw, distw,
                            static_cast<bf16_t *>(d_out), (long long)(2 * p->ld_out), (long long)(2 * p->dist_out),
-                           (int)p->ncols, p->colmax, col_exp, (long long)p->ncols);
+                           (int)p->ncols, p->colmax, col_exp, (long long)p->ncols, tout);
     HIPCHK(hipGetLastError());
-    if (p->timed) HIPCHK(hipEventRecord(p->ev[2], p->stream));
-    p->ran = p->timed;
+    p->ran = p->stamps != nullptr;
     p->col_split = w->four_step && !w->col_long;
     p->col_first = false;
     p->h2d = p->d2h = 0.0;
@@ -1550,6 +1618,7 @@ void split_range(int lgx, int &lo, int &hi)
 // If the temporary spectrum cannot be allocated the default split stays.
 int tune_split(hpxfft_plan_s *p)
 {
+    if (int rc = alloc_events(p)) return rc;
     int lo, hi;
     split_range(p->lgx, lo, hi);
     if (lo >= hi) return HPXFFT_OK;
@@ -1582,11 +1651,11 @@ int tune_split(hpxfft_plan_s *p)
         if (rc == HPXFFT_OK) e = hipEventRecord(p->ev[0], p->stream);
         for (int r = 0; r < REPS && rc == HPXFFT_OK && e == hipSuccess; ++r)
             rc = run_columns(p, tmp, tmp, false, s16 ? p->col_exp_own : nullptr);
-        if (rc == HPXFFT_OK && e == hipSuccess) e = hipEventRecord(p->ev[2], p->stream);
-        if (rc == HPXFFT_OK && e == hipSuccess) e = hipEventSynchronize(p->ev[2]);
+        if (rc == HPXFFT_OK && e == hipSuccess) e = hipEventRecord(p->ev[1], p->stream);
+        if (rc == HPXFFT_OK && e == hipSuccess) e = hipEventSynchronize(p->ev[1]);
         if (rc == HPXFFT_OK && e == hipSuccess)
         {
-            const double ms = elapsed(p->ev[0], p->ev[2]) * 1e3 / REPS;
+            const double ms = elapsed(p->ev[0], p->ev[1]) * 1e3 / REPS;
             (p->col_long ? p->long_ms : p->split_ms[l]) = ms;
             if (best_ms == 0.0 || ms < best_ms)
             {
@@ -1609,7 +1678,7 @@ int tune_split(hpxfft_plan_s *p)
 // measure effort, one-level general rows / columns whose radices allow it:
 // time the forward transform with the ping-pong and the in-place stages on
 // zeroed buffers of the plan's layout (the row and column passes are timed
-// apart by the exec's own events) and keep the faster form of each pass.
+// apart by the exec's own stamps) and keep the faster form of each pass.
 // If the buffers cannot be allocated the estimate stays.
 int tune_gen_ip(hpxfft_plan_s *p)
 {
@@ -1639,11 +1708,12 @@ int tune_gen_ip(hpxfft_plan_s *p)
         for (int r = 0; r <= REPS && rc == HPXFFT_OK && e == hipSuccess; ++r)   // r = 0: warm-up
         {
             rc = exec_forward(p, in, out, nullptr, nullptr);
-            if (rc == HPXFFT_OK) e = hipEventSynchronize(p->ev[2]);
-            if (rc == HPXFFT_OK && e == hipSuccess && r > 0)
+            phase_times pt{};
+            if (rc == HPXFFT_OK) rc = read_times(p, pt);
+            if (rc == HPXFFT_OK && r > 0)
             {
-                row_s += elapsed(p->ev[0], p->ev[1]);
-                col_s += elapsed(p->ev[1], p->ev[2]);
+                row_s += pt.first;
+                col_s += pt.second;
             }
         }
         p->gip_ms[0][ip] = row_ok ? row_s * 1e3 / REPS : 0.0;
@@ -1667,6 +1737,7 @@ int tune_gen_ip(hpxfft_plan_s *p)
 // keep the faster (the scratch of the two-level form is freed if unused)
 int tune_gen_columns(hpxfft_plan_s *p)
 {
+    if (int rc = alloc_events(p)) return rc;
     const size_t bytes = p->batch * p->dist_out * 2 * storage_bytes(p->prec);
     void *tmp = nullptr;
     if (hipMalloc(&tmp, bytes) != hipSuccess)
@@ -1684,9 +1755,9 @@ int tune_gen_columns(hpxfft_plan_s *p)
         rc = run_columns(p, tmp, tmp, false, nullptr);   // warm-up
         if (rc == HPXFFT_OK) e = hipEventRecord(p->ev[0], p->stream);
         for (int r = 0; r < REPS && rc == HPXFFT_OK && e == hipSuccess; ++r) rc = run_columns(p, tmp, tmp, false, nullptr);
-        if (rc == HPXFFT_OK && e == hipSuccess) e = hipEventRecord(p->ev[2], p->stream);
-        if (rc == HPXFFT_OK && e == hipSuccess) e = hipEventSynchronize(p->ev[2]);
-        if (rc == HPXFFT_OK && e == hipSuccess) p->gcol_ms[two] = elapsed(p->ev[0], p->ev[2]) * 1e3 / REPS;
+        if (rc == HPXFFT_OK && e == hipSuccess) e = hipEventRecord(p->ev[1], p->stream);
+        if (rc == HPXFFT_OK && e == hipSuccess) e = hipEventSynchronize(p->ev[1]);
+        if (rc == HPXFFT_OK && e == hipSuccess) p->gcol_ms[two] = elapsed(p->ev[0], p->ev[1]) * 1e3 / REPS;
     }
     (void)hipStreamSynchronize(p->stream);
     (void)hipFree(tmp);
@@ -1708,6 +1779,7 @@ int tune_gen_columns(hpxfft_plan_s *p)
 // ahead on MI355X).  If the buffers cannot be allocated the default stays.
 int tune_rows(hpxfft_plan_s *p)
 {
+    if (int rc = alloc_events(p)) return rc;
     if (p->gen_row || !row_pair_covers(p->prec, p->lgL)) return HPXFFT_OK;
     const size_t sb = storage_bytes(p->prec);
     const size_t bin = p->batch * p->dist_in * sb, bout = p->batch * p->dist_out * 2 * sb;
@@ -1741,11 +1813,11 @@ int tune_rows(hpxfft_plan_s *p)
         e = launch_rows_pow2(p, r, kind);   // warm-up
         if (e == hipSuccess) e = hipEventRecord(p->ev[0], p->stream);
         for (int i = 0; i < REPS && e == hipSuccess; ++i) e = launch_rows_pow2(p, r, kind);
-        if (e == hipSuccess) e = hipEventRecord(p->ev[2], p->stream);
-        if (e == hipSuccess) e = hipEventSynchronize(p->ev[2]);
+        if (e == hipSuccess) e = hipEventRecord(p->ev[1], p->stream);
+        if (e == hipSuccess) e = hipEventSynchronize(p->ev[1]);
         if (e == hipSuccess)
         {
-            p->row_ms[kind] = elapsed(p->ev[0], p->ev[2]) * 1e3 / REPS;
+            p->row_ms[kind] = elapsed(p->ev[0], p->ev[1]) * 1e3 / REPS;
             if (kind == 0 || p->row_ms[kind] < best)
             {
                 best = p->row_ms[kind];
@@ -1813,7 +1885,7 @@ int plan_wide16(hpxfft_plan_s *p)
     HIPCHK(hipMalloc(&p->wide_ws, sizeof(float) * p->batch * w->dist_in));
     HIPCHK(hipMalloc(&p->colmax, sizeof(unsigned) * p->ncols * p->batch));
     HIPCHK(hipMalloc(&p->col_exp_own, sizeof(int) * p->ncols * p->batch));
-    if (int rc = alloc_events(p)) return rc;
+    if (int rc = alloc_timing(p)) return rc;
     p->plan_flops = w->plan_flops;
     return HPXFFT_OK;
 }
@@ -2064,7 +2136,7 @@ int plan_common(hpxfft_plan_s *p)
             HIPCHK(hipMalloc(&p->colmax, sizeof(unsigned) * p->ncols * p->batch));
         }
     }
-    if (int rc = alloc_events(p)) return rc;
+    if (int rc = alloc_timing(p)) return rc;
     if (p->four_step && p->effort >= HPXFFT_MEASURE)
         if (int rc = tune_split(p)) return rc;
     if (p->effort >= HPXFFT_PATIENT)
@@ -2090,6 +2162,7 @@ void free_plan(hpxfft_plan_s *p)
     else (void)hipDeviceSynchronize();
     for (auto &e : p->ev)
         if (e) (void)hipEventDestroy(e);
+    free_timing(p);
     (void)hipFree(p->scratch);
     (void)hipFree(p->mid_exp);
     (void)hipFree(p->colpart);
@@ -2250,7 +2323,7 @@ int hpxfft_exec_r2c_2d_noalloc(size_t nx, size_t ny, size_t ld_in, size_t ld_out
                                                  "and 2 <= Ny <= 32768 (got " + dims + ")");
         if (ld_in < ny || ld_in % 2 || ld_out < ny / 2 + 1)
             return fail(HPXFFT_INVALID_ARG, "layout: need an even ld_in >= Ny and ld_out >= Ny/2+1");
-        hpxfft_plan_s p;   // the plan's fields only: no events, no device memory of its own
+        hpxfft_plan_s p;   // the plan's fields only: no stamps, no device memory of its own
         p.nx = nx;
         p.ny = ny;
         p.ld_in = ld_in;
@@ -2259,7 +2332,6 @@ int hpxfft_exec_r2c_2d_noalloc(size_t nx, size_t ny, size_t ld_in, size_t ld_out
         p.dist_out = nx * ld_out;
         p.prec = precision;
         p.stream = static_cast<hipStream_t>(stream);
-        p.timed = false;
         p.lgx = ilog2(nx);
         p.lgL = ilog2(ny / 2);
         p.ncols = ny / 2 + 1;
@@ -2314,17 +2386,18 @@ int hpxfft_exec_r2c_2d_host(hpxfft_plan plan, double *inout)
             HIPCHK(hipMalloc(&plan->host_buf, bytes));
             plan->host_bytes = bytes;
         }
-        scoped_event e0, e1;   // destroyed on every return path
-        HIPCHK(hipEventCreate(&e0.ev));
-        HIPCHK(hipEventCreate(&e1.ev));
+        scoped_event e0, e1, in_done, out_start;   // destroyed on every return path
+        for (scoped_event *e : {&e0, &e1, &in_done, &out_start}) HIPCHK(hipEventCreate(&e->ev));
         HIPCHK(hipEventRecord(e0.ev, plan->stream));
         HIPCHK(hipMemcpyAsync(plan->host_buf, inout, bytes, hipMemcpyHostToDevice, plan->stream));
+        HIPCHK(hipEventRecord(in_done.ev, plan->stream));
         if (int rc = exec_forward(plan, plan->host_buf, plan->host_buf, nullptr, nullptr)) return rc;
+        HIPCHK(hipEventRecord(out_start.ev, plan->stream));
         HIPCHK(hipMemcpyAsync(inout, plan->host_buf, bytes, hipMemcpyDeviceToHost, plan->stream));
         HIPCHK(hipEventRecord(e1.ev, plan->stream));
         HIPCHK(hipEventSynchronize(e1.ev));
-        plan->h2d = elapsed(e0.ev, plan->ev[0]);
-        plan->d2h = elapsed(plan->ev[2], e1.ev);
+        plan->h2d = elapsed(e0.ev, in_done.ev);
+        plan->d2h = elapsed(out_start.ev, e1.ev);
         return HPXFFT_OK;
     });
 }
@@ -2351,11 +2424,11 @@ int exec_backward(hpxfft_plan_s *plan, const void *d_spec, void *d_real, bool ha
         HIPCHK(hipMalloc(&plan->adj_work, bytes));
         plan->adj_bytes = bytes;
     }
-    if (int rc = alloc_events(plan)) return rc;
-    HIPCHK(hipEventRecord(plan->ev[0], plan->stream));
-    if (int rc = run_columns(plan, d_spec, plan->adj_work, true, nullptr, plan->ev[3])) return rc;
-    HIPCHK(hipEventRecord(plan->ev[1], plan->stream));
+    if (int rc = run_columns(plan, d_spec, plan->adj_work, true, nullptr, {stamp_start(plan), nullptr},
+                             stamp_at(plan, ST_SPLIT)))
+        return rc;
     RowArgs r{};
+    r.ts = {stamp_at(plan, ST_MID), stamp_ends(plan)};
     r.in = plan->adj_work;
     r.out = d_real;
     r.ld_in = (long long)(2 * plan->ld_out);
@@ -2369,7 +2442,7 @@ int exec_backward(hpxfft_plan_s *plan, const void *d_spec, void *d_real, bool ha
     r.stw32 = plan->tabs.stw32;
     if (plan->g2r.on)
     {
-        if (int rc = run_rows_2level(plan, nullptr, d_real, plan->adj_work, nullptr, true, halve)) return rc;
+        if (int rc = run_rows_2level(plan, nullptr, d_real, plan->adj_work, nullptr, true, halve, r.ts)) return rc;
     }
     else if (plan->gen_row)
     {
@@ -2399,7 +2472,6 @@ int exec_backward(hpxfft_plan_s *plan, const void *d_spec, void *d_real, bool ha
         const unsigned gx = (unsigned)((plan->nx + rg.nseq - 1) / rg.nseq);
         HIPCHK(row_c2r(plan->prec, plan->lgL, halve, r, gx, (unsigned)plan->batch, plan->stream));
     }
-    HIPCHK(hipEventRecord(plan->ev[2], plan->stream));
     plan->ran = true;
     plan->col_split = plan->four_step && !plan->col_long;
     plan->col_first = true;
@@ -2435,29 +2507,17 @@ int hpxfft_get_measurement(hpxfft_plan plan, const char *key, double *value)
         else if (k == "first_trans" || k == "second_trans") v = 0.0;
         else if (k == "h2d") v = plan->h2d;
         else if (k == "d2h") v = plan->d2h;
-        else if (k == "total" || k == "first_fftw" || k == "second_fftw")
+        else if (k == "total" || k == "first_fftw" || k == "second_fftw" || k == "column_a" || k == "column_b")
         {
-            if (plan->ran)
+            // column_a, column_b: the two launches of a four-step column pass (0 when the last run had none)
+            const bool split = k == "column_a" || k == "column_b";
+            if (plan->ran && (!split || plan->col_split))
             {
                 device_guard g(plan->device);
-                HIPCHK(hipEventSynchronize(plan->ev[2]));
-                if (k == "total") v = elapsed(plan->ev[0], plan->ev[2]);
-                else if (k == "first_fftw") v = elapsed(plan->ev[0], plan->ev[1]);
-                else v = elapsed(plan->ev[1], plan->ev[2]);
-            }
-        }
-        else if (k == "column_a" || k == "column_b")
-        {
-            // the two launches of a four-step column pass (0 when the last run had no split)
-            if (plan->ran && plan->col_split)
-            {
-                device_guard g(plan->device);
-                HIPCHK(hipEventSynchronize(plan->ev[2]));
-                // forward: rows ev0..ev1, columns ev1..ev3..ev2; backward: columns ev0..ev3..ev1, rows ev1..ev2
-                if (plan->col_first)
-                    v = k == "column_a" ? elapsed(plan->ev[0], plan->ev[3]) : elapsed(plan->ev[3], plan->ev[1]);
-                else
-                    v = k == "column_a" ? elapsed(plan->ev[1], plan->ev[3]) : elapsed(plan->ev[3], plan->ev[2]);
+                phase_times t{};
+                if (int rc = read_times(plan, t)) return rc;
+                v = k == "total" ? t.total : k == "first_fftw" ? t.first : k == "second_fftw" ? t.second
+                    : k == "column_a" ? t.split_a : t.split_b;
             }
         }
         else
@@ -2516,17 +2576,18 @@ namespace {
 int batched_run(hpxfft_plan_s *p, int cfg_row, int cfg_col)
 {
     const int cfg[2] = {cfg_row, cfg_col};
+    // both phases' tickets in one clear
+    hipLaunchKernelGGL(hpxfft_dev::zero_u32_kernel<0>, dim3(1), dim3(64), 0, p->stream, p->bticket,
+                       (long long)(2 * BATCH_QUEUES));
+    HIPCHK(hipGetLastError());
     for (int ph = 0; ph < 2; ++ph)
     {
         unsigned *tk = p->bticket + ph * BATCH_QUEUES;
-        hipLaunchKernelGGL(hpxfft_dev::zero_u32_kernel<0>, dim3(1), dim3(64), 0, p->stream, tk,
-                           (long long)BATCH_QUEUES);
-        HIPCHK(hipGetLastError());
         const int c = cfg[ph];
         const int nb = std::min(p->bblocks[ph][c], std::max(1, p->bntasks[ph][c]));
         HIPCHK(batched_launch(ph, c, p->bgrids, p->btasks[ph][c], p->bntasks[ph][c], tk, p->tabs.tw32, nb,
+                              stamp_at(p, ph == 0 ? ST_START : ST_MID), ph == 0 ? nullptr : stamp_at(p, ST_END),
                               p->stream));
-        if (ph == 0) HIPCHK(hipEventRecord(p->ev[1], p->stream));
     }
     return HPXFFT_OK;
 }
@@ -2598,7 +2659,7 @@ int batched_autotune(hpxfft_plan_s *p)
                                        (long long)BATCH_QUEUES);
                     (void)hipEventRecord(a, p->stream);
                     if (batched_launch(ph, c, p->bgrids, p->btasks[ph][c], p->bntasks[ph][c], tk, p->tabs.tw32, nb,
-                                       p->stream) != hipSuccess)
+                                       nullptr, nullptr, p->stream) != hipSuccess)
                         rc = fail(HPXFFT_HIP_ERROR, "batched autotune launch failed");
                     (void)hipEventRecord(b, p->stream);
                     (void)hipEventSynchronize(b);
@@ -2635,7 +2696,7 @@ int plan_batched(hpxfft_plan_s *p)
     }
     if (int rc = check_device(p->device)) return rc;
     if (int rc = get_tables(p->device, p->tabs)) return rc;
-    if (int rc = alloc_events(p)) return rc;
+    if (int rc = alloc_timing(p)) return rc;
     const size_t n = p->bnx.size();
     HIPCHK(hipMalloc(&p->bgrids, batched_grid_desc_bytes() * n));
     HIPCHK(hipHostMalloc(&p->bstage, 2 * batched_grid_desc_bytes() * n, hipHostMallocDefault));
@@ -2784,9 +2845,7 @@ int hpxfft_exec_r2c_2d_batched(hpxfft_plan plan, void *const *d_grids)
         if (!d_grids) return fail(HPXFFT_INVALID_ARG, "null grid pointer array");
         device_guard g(plan->device);
         if (int rc = batched_upload_grids(plan, d_grids)) return rc;
-        HIPCHK(hipEventRecord(plan->ev[0], plan->stream));
         if (int rc = batched_run(plan, plan->bcfg[0], plan->bcfg[1])) return rc;
-        HIPCHK(hipEventRecord(plan->ev[2], plan->stream));
         plan->ran = true;
         plan->col_split = false;
         return HPXFFT_OK;

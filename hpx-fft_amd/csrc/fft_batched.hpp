@@ -126,8 +126,9 @@ __device__ __attribute__((noinline)) void brow_task(const BGrid &g, int row0, co
 template <int CFG>
 __global__ void __launch_bounds__(brow_cfg<CFG>::NT)
 batched_rows_kernel(const BGrid *__restrict__ grids, const BTask *__restrict__ tasks, int ntasks,
-                    unsigned *ticket, const float *__restrict__ tw32)
+                    unsigned *ticket, const float *__restrict__ tw32, Stamps ts)
 {
+    const unsigned long long t_start = stamp_now(ts, ntasks);
     __shared__ cpx<float> lds[brow_lds<CFG>()];
     __shared__ unsigned slot;
     for (;;)
@@ -147,6 +148,7 @@ batched_rows_kernel(const BGrid *__restrict__ grids, const BTask *__restrict__ t
         }
         __syncthreads();   // LDS reuse by the next task
     }
+    stamp_first(ts, t_start);
 }
 
 template <int CFG, int LGX>
@@ -171,8 +173,9 @@ __device__ __attribute__((noinline)) void bcol_task(const BGrid &g, int strip, c
 template <int CFG>
 __global__ void __launch_bounds__(bcol_cfg<CFG>::NT)
 batched_cols_kernel(const BGrid *__restrict__ grids, const BTask *__restrict__ tasks, int ntasks,
-                    unsigned *ticket, const float *__restrict__ tw32)
+                    unsigned *ticket, const float *__restrict__ tw32, Stamps ts)
 {
+    const unsigned long long t_start = stamp_now(ts, ntasks);
     __shared__ cpx<float> lds[bcol_lds<CFG>()];
     __shared__ unsigned slot;
     for (;;)
@@ -192,6 +195,7 @@ batched_cols_kernel(const BGrid *__restrict__ grids, const BTask *__restrict__ t
         }
         __syncthreads();
     }
+    stamp(ts, t_start);
 }
 
 }   // namespace hpxfft_dev

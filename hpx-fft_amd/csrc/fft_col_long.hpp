@@ -110,6 +110,7 @@ __global__ void __launch_bounds__(NTH, 4) col_long_kernel(ColArgs a)
     using C = collong<T, LG, NTH>;
     constexpr int W = C::W, JT = C::JT, M = C::M, RL = C::RL, NSL = C::NSL, NB = C::NB;
     __shared__ T lds[C::LP * W];
+    const unsigned long long t_start = stamp_now(a.ts, a.ncols);
     const int t = threadIdx.x, w = t % W, jj = t / W;
     const blk3 bk = xcd_block();   // neighbouring strips share lines: one XCD
     const int c = bk.x * W + w;
@@ -148,6 +149,7 @@ __global__ void __launch_bounds__(NTH, 4) col_long_kernel(ColArgs a)
         const cpx<T> z = v[u];
         stor<T>::st(out + 2 * a.pitch * ((u / R) * JT + (u % R) * STR), CONJ ? conjc(z) : z);
     }
+    stamp(a.ts, t_start);
 }
 
 }   // namespace hpxfft_dev

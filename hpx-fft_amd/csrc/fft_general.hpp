@@ -709,6 +709,7 @@ __global__ void __launch_bounds__(NTMAX) gen_row_r2c_kernel(RowArgs a, GenPlan g
                                                             const cpx<double> *tab2, int nseq)
 {
     constexpr bool S16 = is16<S>();
+    const unsigned long long t_start = stamp_now(a.ts, a.nrows);
     cpx<T> *buf = gen_lds<T>();
     const int t = threadIdx.x, L = g.len, ST = g.n;
     unsigned *smax = reinterpret_cast<unsigned *>(buf + gen_nbuf(g) * nseq * ST);
@@ -809,6 +810,7 @@ __global__ void __launch_bounds__(NTMAX) gen_row_r2c_kernel(RowArgs a, GenPlan g
             if (2 * k != L) stor<S>::st(o + 2 * (L - k), x1);
         }
     }
+    stamp_first(a.ts, t_start);
 }
 
 // Column c2c of any Nx: a workgroup takes W adjacent columns over all Nx rows
@@ -824,6 +826,7 @@ template <typename T, typename S, bool CONJ, int NTMAX = GEN_NT>
 __global__ void __launch_bounds__(NTMAX) gen_col_kernel(ColArgs a, GenPlan g, const cpx<double> *tab, int W)
 {
     constexpr bool S16 = is16<S>();
+    const unsigned long long t_start = stamp_now(a.ts, a.ncols);
     cpx<T> *buf = gen_lds<T>();
     const int t = threadIdx.x, n = g.len, ST = g.n;
     unsigned *smax = reinterpret_cast<unsigned *>(buf + gen_nbuf(g) * W * ST);
@@ -884,6 +887,7 @@ __global__ void __launch_bounds__(NTMAX) gen_col_kernel(ColArgs a, GenPlan g, co
         }
         stor<S>::st(dst + 2 * ((long long)e * a.pitch + col0 + w), CONJ ? conjc(z) : z);
     }
+    stamp(a.ts, t_start);
 }
 
 // Row c2r of any even Ny (the row half of the adjoint when HALVE, the
@@ -896,6 +900,7 @@ template <typename T, bool HALVE, int NTMAX = GEN_NT>
 __global__ void __launch_bounds__(NTMAX) gen_row_c2r_kernel(RowArgs a, GenPlan g, const cpx<double> *tabL,
                                                             const cpx<double> *tab2, int nseq)
 {
+    const unsigned long long t_start = stamp_now(a.ts, a.nrows);
     cpx<T> *buf = gen_lds<T>();
     const int t = threadIdx.x, L = g.len, ST = g.n;
     const long long b = blockIdx.y;
@@ -936,6 +941,7 @@ __global__ void __launch_bounds__(NTMAX) gen_row_c2r_kernel(RowArgs a, GenPlan g
         const cpx<T> u = U[s * ST + e];
         stor<T>::st(out + s * a.ld_out + 2 * e, cpx<T>{u.x, -u.y});
     }
+    stamp(a.ts, t_start);
 }
 
 }   // namespace hpxfft_dev
@@ -982,6 +988,7 @@ struct GenStride
     // table split at chirp_shift; blue_conj: conjugate the pass-3 result
     int blue_in, blue_out, blue_n, blue_p, blue_conj, chirp_shift;
     const void *chirp;
+    Stamps ts;
 };
 
 // w_n^m from a table split at s (lo[i] = w_n^i, i < 2^s, then hi[j] = w_n^{j 2^s}),
@@ -1024,6 +1031,7 @@ template <typename T, bool GX = false, int NTMAX = GEN_NT>
 __global__ void __launch_bounds__(NTMAX) gen_strided_kernel(GenStride a, GenPlan g, const cpx<double> *tab,
                                                             const cpx<double> *twt, const cpx<double> *tab2, int W)
 {
+    const unsigned long long t_start = stamp_now(a.ts, a.ncols);
     cpx<T> *buf = gen_lds<T>();
     const int t = threadIdx.x, n = g.len, ST = g.n;
     const int col0 = xcd_order((int)blockIdx.x, (int)gridDim.x) * W;
@@ -1098,6 +1106,7 @@ __global__ void __launch_bounds__(NTMAX) gen_strided_kernel(GenStride a, GenPlan
         }
         stor<T>::st(dst + 2 * ((long long)k * a.out_seq + (long long)w * a.out_col), z);
     }
+    stamp(a.ts, t_start);
 }
 
 // Bluestein pass 2 (see GenStride): W sequences of P points (e = m1) per
@@ -1253,14 +1262,16 @@ __global__ void __launch_bounds__(256) gen_split_kernel(void *spec, long long ro
 template <typename S>
 __global__ void __launch_bounds__(256) wide_in_kernel(const S *in, long long ld_in, long long dist_in,
                                                        const int *in_exp, long long exp_dist, float *ws,
-                                                       long long ld_ws, long long dist_ws, int pairs)
+                                                       long long ld_ws, long long dist_ws, int pairs, Stamps ts)
 {
+    const unsigned long long t_start = stamp_now(ts, pairs);
     const int j = (int)(blockIdx.x * blockDim.x + threadIdx.x);
     if (j >= pairs) return;
     const long long b = blockIdx.z, row = blockIdx.y;
     cpx<float> z = stor<S>::ld(in + b * dist_in + row * ld_in + 2 * j);
     if (in_exp) z = scal(z, ldexpf(1.0f, -in_exp[b * exp_dist + row]));
     stor<float>::st(ws + b * dist_ws + row * ld_ws + 2 * j, z);
+    stamp_first(ts, t_start);
 }
 
 // the largest component of each spectrum column over `rows` rows per block
@@ -1285,7 +1296,7 @@ __global__ void __launch_bounds__(256) wide_colmax_kernel(const float *ws, long 
 template <typename S>
 __global__ void __launch_bounds__(256) wide_out_kernel(const float *ws, long long ld_ws, long long dist_ws, S *out,
                                                         long long ld_out, long long dist_out, int ncols,
-                                                        const unsigned *colmax, int *col_exp, long long cexp_dist)
+                                                        const unsigned *colmax, int *col_exp, long long cexp_dist, Stamps ts)
 {
     const int c = (int)(blockIdx.x * blockDim.x + threadIdx.x);
     if (c >= ncols) return;
@@ -1294,6 +1305,7 @@ __global__ void __launch_bounds__(256) wide_out_kernel(const float *ws, long lon
     const cpx<float> z = stor<float>::ld(ws + b * dist_ws + row * ld_ws + 2 * c);
     stor<S>::st(out + b * dist_out + row * ld_out + 2 * c, scal(z, ldexpf(1.0f, e)));
     if (row == 0 && col_exp) col_exp[b * cexp_dist + c] = e;
+    stamp(ts, 0);
 }
 
 }   // namespace hpxfft_dev

@@ -70,6 +70,7 @@ struct RowArgs
     const int *in_exp;     // optional per-row input exponent (value = stored * 2^-e)
     int *out_exp;          // 16-bit outputs: per-row exponent written here
     long long exp_dist;    // between grids, for in_exp/out_exp
+    Stamps ts;
 };
 
 // column-pass arguments; MODE 0 = direct column kernel, 1 = four-step phase A
@@ -95,6 +96,7 @@ struct ColArgs
     int *out_exp;          // 16-bit outputs (MODE 0,2): per-column exponent
     long long rexp_dist;   // between grids for row_exp
     long long cexp_dist;   // between grids for out_exp
+    Stamps ts;
 };
 
 template <typename S> constexpr bool is16() { return sizeof(S) == 2; }
@@ -277,8 +279,10 @@ row_r2c_kernel(RowArgs a)
     using EN = Engine<T, L, E, NSEQ, false, SPLIT>;
     __shared__ typename EN::lds_t lds[EN::LDS_ELEMS];
     __shared__ unsigned smax[is16<SO>() ? NSEQ : 1];
+    const unsigned long long t_start = stamp_now(a.ts, a.nrows);
     const blk3 bk = xcd_block();
     row_r2c_body<T, SI, SO, L, E, NSEQ, SPLIT>(a, bk.y, bk.x * NSEQ, lds, smax);
+    stamp_first(a.ts, t_start);
 }
 
 // ---------------------------------------------------------------------------
@@ -388,8 +392,10 @@ col_kernel(ColArgs a)
     using EN = Engine<T, L, E, W, true, SPLIT>;
     __shared__ typename EN::lds_t lds[EN::LDS_ELEMS];
     __shared__ unsigned smax[is16<S>() ? W : 1];
+    const unsigned long long t_start = stamp_now(a.ts, a.ncols);
     const blk3 bk = xcd_block();
     col_body<T, S, S, L, E, W, SPLIT, CONJ>(a, bk.z, bk.x, lds, smax);
+    stamp(a.ts, t_start);
 }
 
 // ---------------------------------------------------------------------------
@@ -416,6 +422,7 @@ row_c2r_kernel(RowArgs a)
 
     __shared__ typename EN::lds_t lds[EN::LDS_ELEMS];
 
+    const unsigned long long t_start = stamp_now(a.ts, a.nrows);
     const int t = threadIdx.x;
     const blk3 bk = xcd_block();
     const long long b = bk.y;
@@ -535,6 +542,7 @@ row_c2r_kernel(RowArgs a)
             stor<SO>::st(out + (long long)row * a.ld_out + 2 * e, cpx<T>{v[x].x, -v[x].y});
         }
     }
+    stamp(a.ts, t_start);
 }
 
 template <int UNUSED = 0> __global__ void zero_u32_kernel(unsigned *p, long long n)

@@ -494,6 +494,7 @@ row_r2c_big_kernel(RowArgs a)
     constexpr int NT = B::NT;
     __shared__ T lds[B::SPLIT ? B::LP : 2 * B::LP];
     __shared__ unsigned smax;
+    const unsigned long long t_start = stamp_now(a.ts, a.nrows);
     const int t = threadIdx.x;
     if (is16<SO>() && t == 0) smax = 0u;   // ordered before its use by the stage barriers
     const int g = xcd_order((int)blockIdx.x, (int)gridDim.x);   // consecutive rows share an XCD
@@ -534,6 +535,7 @@ row_r2c_big_kernel(RowArgs a)
     big_row_body<T, SO, LG, NB>(v, lds, reinterpret_cast<const cpx<T> *>(a.tw),
                                 reinterpret_cast<const cpx<double> *>(a.stw64),
                                 reinterpret_cast<const cpx<T> *>(a.stw32), orow, t, &smax, oexp);
+    stamp_first(a.ts, t_start);
 }
 
 // Backward rows of 2^11, 2^13 and 2^14 complex points on the radix-16 stages
@@ -566,6 +568,7 @@ row_c2r_big_kernel(RowArgs a)
     constexpr int NF = NSL / NT;                       // last-stage butterflies per thread
     static_assert(NSL % NT == 0, "last-stage butterflies divide among the threads");
     __shared__ T lds[B::SPLIT ? B::LP : 2 * B::LP];
+    const unsigned long long t_start = stamp_now(a.ts, a.nrows);
     const int t = threadIdx.x;
     const int g = xcd_order((int)blockIdx.x, (int)gridDim.x);   // consecutive rows share an XCD
     const int bat = g / a.nrows, row = g - bat * a.nrows;
@@ -699,6 +702,7 @@ row_c2r_big_kernel(RowArgs a)
         for (int q = 0; q < RL; ++q)
             stor<S>::st(orow + 2 * (j + q * NSL), cpx<T>{f[i][q].x, -f[i][q].y});
     }
+    stamp(a.ts, t_start);
 }
 
 }   // namespace hpxfft_dev

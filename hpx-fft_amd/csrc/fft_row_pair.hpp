@@ -169,6 +169,7 @@ __global__ void __launch_bounds__((1 << LG) / 32, 4) row_r2c_pair_kernel(RowArgs
     constexpr int S = PR::S, NB = PR::NB, NP = PR::NP, NT = PR::NT, RL = PR::RL, NPAIR = PR::NPAIR;
     __shared__ T lds[PR::LP];
     __shared__ unsigned smax;
+    const unsigned long long t_start = stamp_now(a.ts, a.nrows);
     const int t = threadIdx.x, p = t >> 1, h = t & 1;
     if (is16<SO>() && t == 0) smax = 0u;   // ordered before its use by the exchange barriers
     const int g = xcd_order((int)blockIdx.x, (int)gridDim.x);   // consecutive rows share an XCD
@@ -329,6 +330,7 @@ __global__ void __launch_bounds__((1 << LG) / 32, 4) row_r2c_pair_kernel(RowArgs
             if (kk[i] != L / 2) stor<SO>::st(orow + 2 * (L - kk[i]), scal(xl[i], sc));
         }
     }
+    stamp_first(a.ts, t_start);
 }
 
 }   // namespace hpxfft_dev

@@ -127,6 +127,7 @@ tile_kernel(ColArgs a)
     __shared__ T lds[SPLIT ? L * W : 2 * L * W];
     __shared__ unsigned smax[S16 ? W : 1];
 
+    const unsigned long long t_start = stamp_now(a.ts, a.ncols);
     const int t = threadIdx.x;
     if constexpr (S16 && MODE == 1)
     {
@@ -340,6 +341,8 @@ tile_kernel(ColArgs a)
             }
         }
     }
+    if constexpr (MODE == 1) stamp_first(a.ts, t_start);
+    else stamp(a.ts, t_start);
 }
 
 }   // namespace hpxfft_dev

@@ -48,24 +48,25 @@ int batched_resident_blocks(int phase, int cfg)
 }
 
 hipError_t batched_launch(int phase, int cfg, const void *grids, const void *tasks, int ntasks, unsigned *ticket,
-                          const float *tw32, int nblocks, hipStream_t s)
+                          const float *tw32, int nblocks, unsigned long long *begin, unsigned long long *end, hipStream_t s)
 {
+    const Stamps ts{begin, end};
     const BGrid *g = reinterpret_cast<const BGrid *>(grids);
     const BTask *t = reinterpret_cast<const BTask *>(tasks);
     const dim3 grid((unsigned)nblocks), block((unsigned)nthreads(phase, cfg));
     if (phase == 0)
     {
-        if (cfg == 0) hipLaunchKernelGGL(batched_rows_kernel<0>, grid, block, 0, s, g, t, ntasks, ticket, tw32);
-        else if (cfg == 1) hipLaunchKernelGGL(batched_rows_kernel<1>, grid, block, 0, s, g, t, ntasks, ticket, tw32);
-        else if (cfg == 2) hipLaunchKernelGGL(batched_rows_kernel<2>, grid, block, 0, s, g, t, ntasks, ticket, tw32);
-        else hipLaunchKernelGGL(batched_rows_kernel<3>, grid, block, 0, s, g, t, ntasks, ticket, tw32);
+        if (cfg == 0) hipLaunchKernelGGL(batched_rows_kernel<0>, grid, block, 0, s, g, t, ntasks, ticket, tw32, ts);
+        else if (cfg == 1) hipLaunchKernelGGL(batched_rows_kernel<1>, grid, block, 0, s, g, t, ntasks, ticket, tw32, ts);
+        else if (cfg == 2) hipLaunchKernelGGL(batched_rows_kernel<2>, grid, block, 0, s, g, t, ntasks, ticket, tw32, ts);
+        else hipLaunchKernelGGL(batched_rows_kernel<3>, grid, block, 0, s, g, t, ntasks, ticket, tw32, ts);
     }
     else
     {
-        if (cfg == 0) hipLaunchKernelGGL(batched_cols_kernel<0>, grid, block, 0, s, g, t, ntasks, ticket, tw32);
-        else if (cfg == 1) hipLaunchKernelGGL(batched_cols_kernel<1>, grid, block, 0, s, g, t, ntasks, ticket, tw32);
-        else if (cfg == 2) hipLaunchKernelGGL(batched_cols_kernel<2>, grid, block, 0, s, g, t, ntasks, ticket, tw32);
-        else hipLaunchKernelGGL(batched_cols_kernel<3>, grid, block, 0, s, g, t, ntasks, ticket, tw32);
+        if (cfg == 0) hipLaunchKernelGGL(batched_cols_kernel<0>, grid, block, 0, s, g, t, ntasks, ticket, tw32, ts);
+        else if (cfg == 1) hipLaunchKernelGGL(batched_cols_kernel<1>, grid, block, 0, s, g, t, ntasks, ticket, tw32, ts);
+        else if (cfg == 2) hipLaunchKernelGGL(batched_cols_kernel<2>, grid, block, 0, s, g, t, ntasks, ticket, tw32, ts);
+        else hipLaunchKernelGGL(batched_cols_kernel<3>, grid, block, 0, s, g, t, ntasks, ticket, tw32, ts);
     }
     return hipGetLastError();
 }

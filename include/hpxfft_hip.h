@@ -149,7 +149,7 @@ int hpxfft_exec_r2c_2d_host(hpxfft_plan plan, double *inout);
  * its work buffer, one spectrum; later calls allocate nothing.
  *
  * Every exec function except the host path and the batched one enqueues
- * only kernels and event records on the plan's stream, so a caller may
+ * only kernels on the plan's stream, so a caller may
  * capture it into a HIP graph once that first allocation is done (make one
  * backward call before capturing a backward one). */
 int hpxfft_exec_r2c_2d_adjoint(hpxfft_plan plan, const void *d_spec, void *d_real);
@@ -174,8 +174,9 @@ int hpxfft_exec_c2r_2d(hpxfft_plan plan, const void *d_spec, void *d_real);
  * exec; 0 otherwise).  The backward execs (adjoint, c2r) run the column
  * pass first: for them "first_fftw" is the column pass and "second_fftw"
  * the row pass; batched plans give their row and column launches.  Unknown keys
- * give 0.0, as std::map::operator[] does in the reference.  Waits for the
- * last exec to finish. */
+ * give 0.0, as std::map::operator[] does in the reference.  The times are
+ * stamped by the launches themselves with the device's wall clock (10 ns); a
+ * replayed graph stamps them too.  Waits for the plan's stream. */
 int hpxfft_get_measurement(hpxfft_plan plan, const char *key, double *value);
 
 /* Replaces hpxfft::shared::loop::write_plans_to_file (loop.cpp:194-212):
@@ -202,7 +203,7 @@ int hpxfft_plan_r2c_2d_batched(hpxfft_plan *plan, size_t count, const size_t *nx
  * by a host-to-device copy on the plan's stream (two pinned staging slots
  * used in turn; the host waits only if the copy made two calls before has
  * not run yet).  With the same pointers as the previous exec, nothing but
- * kernels and event records is enqueued, so such a call may be captured
+ * kernels is enqueued, so such a call may be captured
  * into a HIP graph; capturing a call with a new pointer set gives
  * HPXFFT_INVALID_ARG. */
 int hpxfft_exec_r2c_2d_batched(hpxfft_plan plan, void *const *d_grids);
