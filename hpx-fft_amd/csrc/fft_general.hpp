@@ -29,7 +29,7 @@
 // natural order to X[k] at pos(k), the product with the kernel spectrum
 // reads that spectrum stored in the same order, and the decimation-in-time
 // stages bring the inverse transform back to natural order.
-// Twiddles and the roots w_r^e = w_n^{e n/r} come from the plan's exact FP64
+// Twiddles and the roots of the generic stage come from the plan's exact FP64
 // table (rounded once for FP32); a register butterfly loads w^k and forms
 // w^{qk} (q < r <= 8) as FP64 powers of it.
 #pragma once
@@ -85,64 +85,78 @@ __device__ __forceinline__ int gdiv(int x, int d, float inv)
     return q;
 }
 
-template <typename T> __device__ __forceinline__ cpx<T> tabv(const cpx<double> *__restrict__ tab, int m)
+// cos and sin of 2 pi e / R for the odd register radices.  Literals (the values
+// that w_n^{e n/R} has in the plan's table): loaded from the table they held up to
+// 24 scalar registers per radix
+template <int R> struct gen_root;
+template <> struct gen_root<3>
 {
-    const cpx<double> w = tab[m];
-    return cpx<T>{(T)w.x, (T)w.y};
-}
+    static constexpr double c[2] = {1.0, -0.5}, s[2] = {0.0, 0.86602540378443864676};
+};
+template <> struct gen_root<5>
+{
+    static constexpr double c[3] = {1.0, 0.30901699437494742410, -0.80901699437494742410};
+    static constexpr double s[3] = {0.0, 0.95105651629515357212, 0.58778525229247312917};
+};
+template <> struct gen_root<7>
+{
+    static constexpr double c[4] = {1.0, 0.62348980185873353053, -0.22252093395631440429, -0.90096886790241912624};
+    static constexpr double s[4] = {0.0, 0.78183148246802980871, 0.97492791218182360702, 0.43388373911755812048};
+};
 
-// DFT of R points in registers, forward sign; w[e] = w_R^e (e >= 1)
-template <typename T, int R> __device__ __forceinline__ void dft_small(cpx<T> *x, const cpx<T> *w)
+// DFT of R points in registers, forward sign.  Odd R: with s_p = x[p] + x[R-p],
+// d_p = x[p] - x[R-p] (p <= H = (R-1)/2), A_o = x[0] + sum_p cos(2 pi p o / R) s_p
+// and B_o = sum_p sin(2 pi p o / R) d_p,
+//   X[o] = A_o - i B_o, X[R-o] = A_o + i B_o:
+// real factors, 36 and 66 FP instructions for R = 5 and 7, against 72 and 156 of the
+// definition's complex products.  The stages are bound by issue, so this is what
+// moved: 9000 x 18000 FP64 4.71 -> 4.00 ms, 3000 x 3000 0.125 -> 0.100 (with
+// gen_unroll below).
+template <typename T, int R> __device__ __forceinline__ void dft_small(cpx<T> *x)
 {
-    if constexpr (R == 2)
-    {
-        const cpx<T> a = x[0], b = x[1];
-        x[0] = a + b;
-        x[1] = a - b;
-    }
-    else if constexpr (R == 4)
-    {
-        const cpx<T> s0 = x[0] + x[2], d0 = x[0] - x[2], s1 = x[1] + x[3], d1 = x[1] - x[3];
-        x[0] = s0 + s1;
-        x[2] = s0 - s1;
-        x[1] = d0 + mul_mi(d1);
-        x[3] = d0 - mul_mi(d1);
-    }
-    else if constexpr (R == 8)
-    {
-        // two 4-point DFTs of the even and odd inputs, X[k] = E[k] + w_8^k O[k],
-        // X[k+4] = E[k] - w_8^k O[k] (w_8 = w[1], w_8^2 = -i, w_8^3 = w[3])
-        cpx<T> e[4] = {x[0], x[2], x[4], x[6]}, o[4] = {x[1], x[3], x[5], x[7]};
-        dft_small<T, 4>(e, w);
-        dft_small<T, 4>(o, w);
-        o[1] = cmul(o[1], w[1]);
-        o[2] = mul_mi(o[2]);
-        o[3] = cmul(o[3], w[3]);
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-        {
-            x[k] = e[k] + o[k];
-            x[k + 4] = e[k] - o[k];
-        }
-    }
+    if constexpr (R == 2) dft2(x);
+    else if constexpr (R == 4) dft4(x);
+    else if constexpr (R == 8) dft8(x);
     else
     {
-        cpx<T> y[R];
+        constexpr int H = (R - 1) / 2;
+        cpx<T> sp[H + 1], dp[H + 1];
+        const cpx<T> x0 = x[0];
 #pragma unroll
-        for (int o = 0; o < R; ++o)
+        for (int p = 1; p <= H; ++p)
         {
-            cpx<T> acc = x[0];
-#pragma unroll
-            for (int q = 1; q < R; ++q)
-            {
-                const int e = (q * o) % R;
-                acc = e == 0 ? acc + x[q] : acc + cmul(x[q], w[e]);
-            }
-            y[o] = acc;
+            sp[p] = x[p] + x[R - p];
+            dp[p] = x[p] - x[R - p];
+            x[0] = x[0] + sp[p];
         }
 #pragma unroll
-        for (int o = 0; o < R; ++o) x[o] = y[o];
+        for (int o = 1; o <= H; ++o)
+        {
+            cpx<T> a = x0, b = {T(0), T(0)};
+#pragma unroll
+            for (int p = 1; p <= H; ++p)
+            {
+                const int e = (p * o) % R;
+                const T c = (T)gen_root<R>::c[e <= H ? e : R - e];
+                const T sn = (T)(e <= H ? gen_root<R>::s[e] : -gen_root<R>::s[R - e]);
+                a = a + scal(sp[p], c);
+                b = p == 1 ? scal(dp[p], sn) : b + scal(dp[p], sn);
+            }
+            const cpx<T> ib = mul_mi(b);   // -i B_o
+            x[o] = a + ib;
+            x[R - o] = a - ib;
+        }
     }
+}
+
+// butterflies of a register stage that a thread takes per iteration.  Two keep more
+// loads in flight; where two FP64 butterflies of radix 7 or 8, or any two in the
+// 1024-thread build, need more than the 128 VGPRs of 4 waves per SIMD, one: with two,
+// 40-50 VGPRs were spilled (2310 x 2310 x 4 FP64 582 -> 507 us, 3000 x 3000 108 ->
+// 100, 9000 x 18000 4570 -> 4000).
+template <typename T, int R, int NTMAX> constexpr int gen_unroll()
+{
+    return sizeof(T) == 8 && (R >= 7 || NTMAX != GEN_NT) ? 1 : 2;
 }
 
 // one Stockham stage of radix R (2, 3, 4, 5, 7, 8) over nseq sequences, A -> B
@@ -151,20 +165,17 @@ __device__ void gen_stage_reg(const cpx<T> *A, cpx<T> *B, int nseq, int n, int N
 {
     const int t = threadIdx.x, m = n / R, nb = nseq * m, tstep = n / (R * Ns);
     const float inv_m = 1.0f / (float)m, inv_ns = 1.0f / (float)Ns;
-    cpx<T> w[R];
-#pragma unroll
-    for (int e = 1; e < R; ++e) w[e] = tabv<T>(tab, e * m);
-    w[0] = cpx<T>{T(1), T(0)};
-    // two butterflies per iteration (independent loads in flight together);
+    // UN butterflies per iteration (independent loads in flight together);
     // twiddles w^{qk} as powers of the one table value w^k, in FP64
+    constexpr int UN = gen_unroll<T, R, NTMAX>();
     const int NTH = gen_nth<NTMAX>();
-    for (int b0 = t; b0 < nb; b0 += 2 * NTH)
+    for (int b0 = t; b0 < nb; b0 += UN * NTH)
     {
-        cpx<T> x[2][R];
-        cpx<double> w1[2];
+        cpx<T> x[UN][R];
+        cpx<double> w1[UN];
         int dst[2] = {-1, -1}, kk[2] = {0, 0};
 #pragma unroll
-        for (int u = 0; u < 2; ++u)
+        for (int u = 0; u < UN; ++u)
         {
             const int b = b0 + u * NTH;
             if (b < nb)
@@ -180,7 +191,7 @@ __device__ void gen_stage_reg(const cpx<T> *A, cpx<T> *B, int nseq, int n, int N
             }
         }
 #pragma unroll
-        for (int u = 0; u < 2; ++u)
+        for (int u = 0; u < UN; ++u)
         {
             if (dst[u] < 0) continue;
             if (kk[u] > 0)
@@ -194,7 +205,7 @@ __device__ void gen_stage_reg(const cpx<T> *A, cpx<T> *B, int nseq, int n, int N
                     x[u][q] = cmul(x[u][q], cpx<T>{(T)wq.x, (T)wq.y});
                 }
             }
-            dft_small<T, R>(x[u], w);
+            dft_small<T, R>(x[u]);
             cpx<T> *dst_p = B + dst[u];
 #pragma unroll
             for (int q = 0; q < R; ++q) dst_p[q * Ns] = x[u][q];
@@ -212,18 +223,15 @@ __device__ void gen_stage_ip(cpx<T> *A, int nseq, int n, int Ls, const cpx<doubl
 {
     const int t = threadIdx.x, m = n / R, nb = nseq * m, tstep = n / (R * Ls);
     const float inv_m = 1.0f / (float)m, inv_ls = 1.0f / (float)Ls;
-    cpx<T> w[R];
-#pragma unroll
-    for (int e = 1; e < R; ++e) w[e] = tabv<T>(tab, e * m);
-    w[0] = cpx<T>{T(1), T(0)};
+    constexpr int UN = gen_unroll<T, R, NTMAX>();
     const int NTH = gen_nth<NTMAX>();
-    for (int b0 = t; b0 < nb; b0 += 2 * NTH)
+    for (int b0 = t; b0 < nb; b0 += UN * NTH)
     {
-        cpx<T> x[2][R];
-        cpx<double> w1[2];
+        cpx<T> x[UN][R];
+        cpx<double> w1[UN];
         int base[2] = {-1, -1}, jj[2] = {0, 0};
 #pragma unroll
-        for (int u = 0; u < 2; ++u)
+        for (int u = 0; u < UN; ++u)
         {
             const int b = b0 + u * NTH;
             if (b < nb)
@@ -238,7 +246,7 @@ __device__ void gen_stage_ip(cpx<T> *A, int nseq, int n, int Ls, const cpx<doubl
             }
         }
 #pragma unroll
-        for (int u = 0; u < 2; ++u)
+        for (int u = 0; u < UN; ++u)
         {
             if (base[u] < 0) continue;
             if (jj[u] > 0)
@@ -252,7 +260,7 @@ __device__ void gen_stage_ip(cpx<T> *A, int nseq, int n, int Ls, const cpx<doubl
                     x[u][q] = cmul(x[u][q], cpx<T>{(T)wq.x, (T)wq.y});
                 }
             }
-            dft_small<T, R>(x[u], w);
+            dft_small<T, R>(x[u]);
             cpx<T> *p = A + base[u];
             if constexpr (POST)
             {
@@ -286,10 +294,6 @@ __device__ void gen_stage_blue_mid(cpx<T> *A, int nseq, int n, const cpx<double>
 {
     const int t = threadIdx.x, per = n / R, nb = nseq * per;
     const float inv_per = 1.0f / (float)per;
-    cpx<T> w[R];
-#pragma unroll
-    for (int e = 1; e < R; ++e) w[e] = tabv<T>(tab, e * per);
-    w[0] = cpx<T>{T(1), T(0)};
     for (int b = t; b < nb; b += gen_nth<NTMAX>())
     {
         const int seq = gdiv(b, per, inv_per), c = b - seq * per;
@@ -297,10 +301,10 @@ __device__ void gen_stage_blue_mid(cpx<T> *A, int nseq, int n, const cpx<double>
         cpx<T> x[R];
 #pragma unroll
         for (int q = 0; q < R; ++q) x[q] = p[q];
-        dft_small<T, R>(x, w);
+        dft_small<T, R>(x);
 #pragma unroll
         for (int q = 0; q < R; ++q) x[q] = conjc(cmul(x[q], tabv<T>(bhp, c * R + q)));
-        dft_small<T, R>(x, w);
+        dft_small<T, R>(x);
 #pragma unroll
         for (int q = 0; q < R; ++q) p[q] = x[q];
     }
@@ -377,18 +381,15 @@ __device__ void gen_stage_dif(cpx<T> *A, int nseq, int n, int Lb, const cpx<doub
 {
     const int t = threadIdx.x, per = n / R, nb = nseq * per, m = Lb / R, tstep = n / Lb;
     const float inv_per = 1.0f / (float)per, inv_m = 1.0f / (float)m;
-    cpx<T> w[R];
-#pragma unroll
-    for (int e = 1; e < R; ++e) w[e] = tabv<T>(tab, e * per);
-    w[0] = cpx<T>{T(1), T(0)};
+    constexpr int UN = gen_unroll<T, R, NTMAX>();
     const int NTH = gen_nth<NTMAX>();
-    for (int b0 = t; b0 < nb; b0 += 2 * NTH)
+    for (int b0 = t; b0 < nb; b0 += UN * NTH)
     {
-        cpx<T> x[2][R];
-        cpx<double> w1[2];
+        cpx<T> x[UN][R];
+        cpx<double> w1[UN];
         int base[2] = {-1, -1}, jj[2] = {0, 0};
 #pragma unroll
-        for (int u = 0; u < 2; ++u)
+        for (int u = 0; u < UN; ++u)
         {
             const int b = b0 + u * NTH;
             if (b < nb)
@@ -417,10 +418,10 @@ __device__ void gen_stage_dif(cpx<T> *A, int nseq, int n, int Lb, const cpx<doub
             }
         }
 #pragma unroll
-        for (int u = 0; u < 2; ++u)
+        for (int u = 0; u < UN; ++u)
         {
             if (base[u] < 0) continue;
-            dft_small<T, R>(x[u], w);
+            dft_small<T, R>(x[u]);
             if (jj[u] > 0)
             {
                 cpx<double> wq = w1[u];
@@ -639,11 +640,8 @@ __device__ void gen_load_first_r(cpx<T> *buf, int nseq, const GenPlan &g, const 
                                  bool s_fast, LD ld)
 {
     const int n = g.n, per = n / R, total = nseq * per;
-    cpx<T> w[R];
-#pragma unroll
-    for (int e = 1; e < R; ++e) w[e] = tabv<T>(tab, e * per);
-    w[0] = cpx<T>{T(1), T(0)};
     const float inv_per = 1.0f / (float)per, inv_ns = 1.0f / (float)nseq;
+#pragma unroll 1
     for (int i = threadIdx.x; i < total; i += gen_nth<NTMAX>())
     {
         int s, e0;
@@ -660,7 +658,7 @@ __device__ void gen_load_first_r(cpx<T> *buf, int nseq, const GenPlan &g, const 
         cpx<T> x[R];
 #pragma unroll
         for (int q = 0; q < R; ++q) x[q] = ld(s, e0 + q * per);
-        dft_small<T, R>(x, w);
+        dft_small<T, R>(x);
         cpx<T> *o = buf + s * n + gen_pos(g, tab, e0);
 #pragma unroll
         for (int q = 0; q < R; ++q) o[q] = x[q];
@@ -705,7 +703,7 @@ template <typename T> __device__ __forceinline__ cpx<T> *gen_lds()
 // e = pick_exp(its largest component), written to out_exp[row], as the
 // power-of-two row kernels do.
 template <typename T, typename S = T, int NTMAX = GEN_NT>
-__global__ void __launch_bounds__(NTMAX) gen_row_r2c_kernel(RowArgs a, GenPlan g, const cpx<double> *tabL,
+__global__ void __launch_bounds__(NTMAX, 4) gen_row_r2c_kernel(RowArgs a, GenPlan g, const cpx<double> *tabL,
                                                             const cpx<double> *tab2, int nseq)
 {
     constexpr bool S16 = is16<S>();
@@ -823,7 +821,7 @@ __global__ void __launch_bounds__(NTMAX) gen_row_r2c_kernel(RowArgs a, GenPlan g
 // 2^-row_exp[row] on load, and column c is stored times 2^e with e =
 // pick_exp(its largest component), written to out_exp[c].
 template <typename T, typename S, bool CONJ, int NTMAX = GEN_NT>
-__global__ void __launch_bounds__(NTMAX) gen_col_kernel(ColArgs a, GenPlan g, const cpx<double> *tab, int W)
+__global__ void __launch_bounds__(NTMAX, 4) gen_col_kernel(ColArgs a, GenPlan g, const cpx<double> *tab, int W)
 {
     constexpr bool S16 = is16<S>();
     const unsigned long long t_start = stamp_now(a.ts, a.ncols);

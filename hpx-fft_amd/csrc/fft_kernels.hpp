@@ -99,6 +99,13 @@ struct ColArgs
     Stamps ts;
 };
 
+// an entry of an exact FP64 table, rounded once for FP32
+template <typename T> __device__ __forceinline__ cpx<T> tabv(const cpx<double> *__restrict__ tab, int m)
+{
+    const cpx<double> w = tab[m];
+    return cpx<T>{(T)w.x, (T)w.y};
+}
+
 template <typename S> constexpr bool is16() { return sizeof(S) == 2; }
 
 // exponent e with max * 2^e in [2^14, 2^15): keeps fp16 clear of overflow
