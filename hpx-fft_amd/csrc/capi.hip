@@ -9,6 +9,7 @@
 #include "launch.hpp"
 #include "fft_general.hpp"
 #include "batched.hpp"
+#include "blue.hpp"
 #include "../../include/hpxfft_hip.h"
 
 #include <chrono>
@@ -504,6 +505,32 @@ bool gen_setup(size_t n, size_t cap, hpxfft_dev::GenPlan &g, size_t ip_cap = 0)
 // whether a plan can run its stages in place
 bool gen_can_ip(const hpxfft_dev::GenPlan &g) { return g.off_r >= 0 || g.off_bp >= 0; }
 
+// Bluestein lengths of one workgroup that run in registers (fft_blue.hpp): FP64 /
+// FP32 plans whose form is the in-place one.  16-bit storage, the ping-pong form
+// that the measure effort times against it, and the sub-lengths of two-level
+// plans stay with the in-LDS kernels.
+bool blue_covers(const hpxfft_plan_s *p, const hpxfft_dev::GenPlan &g)
+{
+    if (g.len == g.n || !g.ip || (p->prec != P_F64 && p->prec != P_F32)) return false;
+    const int lg = ilog2((size_t)g.n);
+    return lg >= hpxfft_dev::BLUE_MIN_LG &&
+           lg <= (p->prec == P_F64 ? hpxfft_dev::BLUE_MAX_LG_F64 : hpxfft_dev::BLUE_MAX_LG_F32);
+}
+
+// their arguments; toff: the plan's table (complex entries)
+hpxfft_dev::BlueArgs blue_args(const hpxfft_plan_s *p, const hpxfft_dev::GenPlan &g, size_t toff)
+{
+    const auto *tab = reinterpret_cast<const hpxfft_dev::cpx<double> *>(p->gen_tab);
+    hpxfft_dev::BlueArgs a{};
+    a.len = g.len;
+    a.stw64 = reinterpret_cast<const hpxfft_dev::cpx<double> *>(p->tabs.stw64);
+    a.tw_L = tw_ptr(p, (size_t)g.n);
+    a.chirp = tab + toff + g.off_c;
+    a.bh = tab + toff + g.off_b;
+    a.tab2 = tab + p->gtab_2;
+    return a;
+}
+
 // the last resort for a one-level length that no other plan covers (a prime
 // factor above 61 that no split avoids): Bluestein's algorithm through an
 // FFT of more than `cap` and at most 2 cap points, held in one LDS buffer
@@ -814,7 +841,8 @@ std::string describe(const hpxfft_plan_s *p)
             os << "    then the r2c split in place (one thread per pair k, Ny/2-k)\n";
     }
     else if (p->gen_row)
-        os << "  row r2c kernel (general length): " << p->ny / 2 << "-point " << gen_method(p->grow) << ", "
+        os << "  row r2c kernel (general length): " << p->ny / 2 << "-point " << gen_method(p->grow)
+           << (blue_covers(p, p->grow) ? "; forward and inverse transform of each sequence in registers, radix 16" : "") << ", "
            << p->gen_rows << " row(s)/workgroup, "
            << gen_threads(gen_lds_bytes(p, p->grow, (size_t)p->gen_rows * p->grow.n, (size_t)p->gen_rows), p->grow)
            << " threads + r2c split\n";
@@ -841,7 +869,8 @@ std::string describe(const hpxfft_plan_s *p)
            << "\n";
     if (p->g2c.on) two_level("column c2c", p->g2c);
     else if (p->gen_col)
-        os << "  column c2c kernel (general length): " << p->nx << "-point " << gen_method(p->gcol) << ", "
+        os << "  column c2c kernel (general length): " << p->nx << "-point " << gen_method(p->gcol)
+           << (blue_covers(p, p->gcol) ? "; forward and inverse transform of each sequence in registers, radix 16" : "") << ", "
            << p->gen_w << " adjacent columns/workgroup\n";
     else if (!p->four_step)
     {
@@ -1376,6 +1405,14 @@ int run_columns(hpxfft_plan_s *p, const void *spec_in, void *spec_out, bool conj
         // general length (F64 / F32; in place for the forward transform)
         a.in = spec_in;
         a.out = spec_out;
+        if (blue_covers(p, p->gcol))
+        {
+            const int lg = ilog2((size_t)p->gcol.n);
+            const auto g = blue_args(p, p->gcol, p->gtab_N);
+            HIPCHK(p->prec == P_F64 ? hpxfft_host::blue_col_f64(lg, conj, a, g, (unsigned)p->batch, p->stream)
+                                    : hpxfft_host::blue_col_f32(lg, conj, a, g, (unsigned)p->batch, p->stream));
+            return HPXFFT_OK;
+        }
         const dim3 grid((unsigned)((p->ncols + p->gen_w - 1) / p->gen_w), (unsigned)p->batch);
         const size_t lds = gen_lds_bytes(p, p->gcol, (size_t)p->gen_w * p->gcol.n, (size_t)p->gen_w);
         const unsigned nt = gen_threads(lds, p->gcol);
@@ -1518,6 +1555,13 @@ int exec_forward(hpxfft_plan_s *p, const void *d_in, void *d_out, const int *in_
     if (p->g2r.on)
     {
         if (int rc = run_rows_2level(p, d_in, nullptr, nullptr, d_out, false, false, r.ts)) return rc;
+    }
+    else if (p->gen_row && blue_covers(p, p->grow))
+    {
+        const int lg = ilog2((size_t)p->grow.n);
+        const auto bg = blue_args(p, p->grow, p->gtab_L);
+        HIPCHK(p->prec == P_F64 ? hpxfft_host::blue_row_r2c_f64(lg, r, bg, (unsigned)p->batch, p->stream)
+                                : hpxfft_host::blue_row_r2c_f32(lg, r, bg, (unsigned)p->batch, p->stream));
     }
     else if (p->gen_row)
     {
@@ -2443,6 +2487,13 @@ int exec_backward(hpxfft_plan_s *plan, const void *d_spec, void *d_real, bool ha
     if (plan->g2r.on)
     {
         if (int rc = run_rows_2level(plan, nullptr, d_real, plan->adj_work, nullptr, true, halve, r.ts)) return rc;
+    }
+    else if (plan->gen_row && blue_covers(plan, plan->grow))
+    {
+        const int lg = ilog2((size_t)plan->grow.n);
+        const auto bg = blue_args(plan, plan->grow, plan->gtab_L);
+        HIPCHK(plan->prec == P_F64 ? hpxfft_host::blue_row_c2r_f64(lg, halve, r, bg, (unsigned)plan->batch, plan->stream)
+                                   : hpxfft_host::blue_row_c2r_f32(lg, halve, r, bg, (unsigned)plan->batch, plan->stream));
     }
     else if (plan->gen_row)
     {

@@ -31,10 +31,12 @@ constexpr int COL_LONG_MIN_LG = 11, COL_LONG_MAX_LG = 12;
 
 template <typename T, int LG, int NTH> struct collong
 {
+    using real = T;
     static constexpr int L = 1 << LG;
     static constexpr int NB = 8 / (int)sizeof(T);               // radix-16 butterflies per thread and stage
     static constexpr int NT = NTH;                               // threads
     static constexpr int W = NT * 16 * NB / L;          // adjacent columns
+    static constexpr int ES = W;                                 // LDS distance of consecutive elements of a column
     static constexpr int M = L / 16;                             // butterflies per column
     static constexpr int JT = NT / W;                   // threads per column
     static constexpr int NR16 = LG / 4;
@@ -46,19 +48,54 @@ template <typename T, int LG, int NTH> struct collong
     static_assert(W >= 1 && JT * NB == M, "threads cover the butterflies");
 };
 
-// exchange: this thread's outputs of radix-16 stage S to LDS, then the inputs of
-// the next stage of radix R2 (element j + r L/R2 of butterfly j = jj + i JT)
-template <typename T, int LG, int NTH, int S, int R2>
-__device__ __forceinline__ void col_long_exchange(cpx<T> *v, T *lds, int jj, int w)
+// dft16 of inputs whose upper half is zero: the first four 4-point DFTs have two
+template <typename T> __device__ __forceinline__ void dft16_half(cpx<T> *a)
 {
-    using C = collong<T, LG, NTH>;
+    const T c = kconst<T>::c8, s = kconst<T>::s8;
+    cpx<T> y[16];
+#pragma unroll
+    for (int n1 = 0; n1 < 4; ++n1)
+    {
+        const cpx<T> b0 = a[n1], b1 = a[n1 + 4], r1 = mul_mi(b1);
+        y[n1 * 4 + 0] = b0 + b1;
+        y[n1 * 4 + 1] = b0 + r1;
+        y[n1 * 4 + 2] = b0 - b1;
+        y[n1 * 4 + 3] = b0 - r1;
+    }
+    y[5] = cmul(y[5], cpx<T>{c, -s});
+    y[6] = mul_w8_1(y[6]);
+    y[7] = cmul(y[7], cpx<T>{s, -c});
+    y[9] = mul_w8_1(y[9]);
+    y[10] = mul_mi(y[10]);
+    y[11] = mul_w8_3(y[11]);
+    y[13] = cmul(y[13], cpx<T>{s, -c});
+    y[14] = mul_w8_3(y[14]);
+    y[15] = cmul(y[15], cpx<T>{-c, s});
+#pragma unroll
+    for (int k2 = 0; k2 < 4; ++k2)
+    {
+        cpx<T> b0 = y[k2], b1 = y[4 + k2], b2 = y[8 + k2], b3 = y[12 + k2];
+        dft4v(b0, b1, b2, b3);
+        a[k2] = b0;
+        a[4 + k2] = b1;
+        a[8 + k2] = b2;
+        a[12 + k2] = b3;
+    }
+}
+
+// exchange: this thread's outputs of radix-16 stage S to LDS, then the inputs of
+// the next stage of radix R2 (element j + r L/R2 of butterfly j = jj + i JT).
+// Element e lies at lds[pad(e) C::ES + w].
+template <typename C, int S, int R2>
+__device__ __forceinline__ void col_long_exchange(cpx<typename C::real> *v, typename C::real *lds, int jj, int w)
+{
     constexpr int NS = C::ns(S), WS = NS == 1 ? 1 : NS + NS / 16, STR = C::L / R2, RS = STR + STR / 16;
     int wb[C::NB];
 #pragma unroll
     for (int b = 0; b < C::NB; ++b)
     {
         const int j = jj + b * C::JT, k = j & (NS - 1);
-        wb[b] = C::pad((j / NS) * 16 * NS + k) * C::W + w;
+        wb[b] = C::pad((j / NS) * 16 * NS + k) * C::ES + w;
     }
 #pragma unroll
     for (int h = 0; h < 2; ++h)
@@ -66,39 +103,61 @@ __device__ __forceinline__ void col_long_exchange(cpx<T> *v, T *lds, int jj, int
 #pragma unroll
         for (int b = 0; b < C::NB; ++b)
 #pragma unroll
-            for (int q = 0; q < 16; ++q) lds[wb[b] + q * WS * C::W] = h ? v[16 * b + q].y : v[16 * b + q].x;
+            for (int q = 0; q < 16; ++q) lds[wb[b] + q * WS * C::ES] = h ? v[16 * b + q].y : v[16 * b + q].x;
         __syncthreads();
 #pragma unroll
         for (int i = 0; i < 16 * C::NB / R2; ++i)
         {
-            const int rb = C::pad(jj + i * C::JT) * C::W + w;
+            const int rb = C::pad(jj + i * C::JT) * C::ES + w;
 #pragma unroll
             for (int r = 0; r < R2; ++r)
             {
-                if (h) v[i * R2 + r].y = lds[rb + r * RS * C::W];
-                else v[i * R2 + r].x = lds[rb + r * RS * C::W];
+                if (h) v[i * R2 + r].y = lds[rb + r * RS * C::ES];
+                else v[i * R2 + r].x = lds[rb + r * RS * C::ES];
             }
         }
         if (h == 0) __syncthreads();
     }
 }
 
-template <typename T, int LG, int NTH, int S>
-__device__ __forceinline__ void col_long_stages(cpx<T> *v, T *lds, const cpx<double> *__restrict__ stw64, int jj, int w)
+// HALF: the inputs 8..15 of each stage-0 butterfly are zero
+template <typename C, int S, bool HALF = false>
+__device__ __forceinline__ void col_long_stages(cpx<typename C::real> *v, typename C::real *lds,
+                                                const cpx<double> *__restrict__ stw64, int jj, int w)
 {
-    using C = collong<T, LG, NTH>;
+    using T = typename C::real;
     constexpr int NS = C::ns(S);
 #pragma unroll
     for (int b = 0; b < C::NB; ++b)
     {
         if constexpr (NS > 1) twiddle16<T, NS>(v + 16 * b, stw64, (jj + b * C::JT) & (NS - 1));
-        dft16(v + 16 * b);
+        if constexpr (HALF) dft16_half(v + 16 * b);
+        else dft16(v + 16 * b);
     }
     if constexpr (S + 1 < C::NR16)
     {
         if constexpr (S > 0) __syncthreads();   // the last exchange's reads
-        col_long_exchange<T, LG, NTH, S, 16>(v, lds, jj, w);
-        col_long_stages<T, LG, NTH, S + 1>(v, lds, stw64, jj, w);
+        col_long_exchange<C, S, 16>(v, lds, jj, w);
+        col_long_stages<C, S + 1>(v, lds, stw64, jj, w);
+    }
+}
+
+// the last stage, radix RL > 1, after its exchange: butterfly j reads
+// j + r NSL, outputs j + q NSL (v[i RL + q], j = jj + i JT); twiddles w_L^{r j}
+template <typename C>
+__device__ __forceinline__ void col_long_last(cpx<typename C::real> *v, typename C::real *lds,
+                                              const cpx<typename C::real> *__restrict__ tw, int jj, int w)
+{
+    using T = typename C::real;
+    constexpr int RL = C::RL;
+    __syncthreads();
+    col_long_exchange<C, C::NR16 - 1, RL>(v, lds, jj, w);
+#pragma unroll
+    for (int i = 0; i < 16 * C::NB / RL; ++i)
+    {
+#pragma unroll
+        for (int r = 1; r < RL; ++r) v[i * RL + r] = cmul(v[i * RL + r], tw[r * (jj + i * C::JT)]);
+        dftR<T, RL>(v + i * RL);
     }
 }
 
@@ -126,21 +185,8 @@ __global__ void __launch_bounds__(NTH, 4) col_long_kernel(ColArgs a)
         cpx<T> z = stor<T>::ld(in + 2 * a.pitch * ((u / 16) * JT + (u % 16) * M));
         v[u] = CONJ ? conjc(z) : z;
     }
-    col_long_stages<T, LG, NTH, 0>(v, lds, reinterpret_cast<const cpx<double> *>(a.stw64), jj, w);
-    if constexpr (RL > 1)
-    {
-        // last stage: butterfly j reads j + r NSL, outputs j + q NSL; twiddles w_L^{r j}
-        __syncthreads();
-        col_long_exchange<T, LG, NTH, C::NR16 - 1, RL>(v, lds, jj, w);
-        const cpx<T> *tw = reinterpret_cast<const cpx<T> *>(a.tw_L);
-#pragma unroll
-        for (int i = 0; i < 16 * NB / RL; ++i)
-        {
-#pragma unroll
-            for (int r = 1; r < RL; ++r) v[i * RL + r] = cmul(v[i * RL + r], tw[r * (jj + i * JT)]);
-            dftR<T, RL>(v + i * RL);
-        }
-    }
+    col_long_stages<C, 0>(v, lds, reinterpret_cast<const cpx<double> *>(a.stw64), jj, w);
+    if constexpr (RL > 1) col_long_last<C>(v, lds, reinterpret_cast<const cpx<T> *>(a.tw_L), jj, w);
     if (!valid) return;
     constexpr int R = RL > 1 ? RL : 16, STR = RL > 1 ? NSL : M;
 #pragma unroll
