@@ -2636,7 +2636,7 @@ int batched_run(hpxfft_plan_s *p, int cfg_row, int cfg_col)
         unsigned *tk = p->bticket + ph * BATCH_QUEUES;
         const int c = cfg[ph];
         const int nb = std::min(p->bblocks[ph][c], std::max(1, p->bntasks[ph][c]));
-        HIPCHK(batched_launch(ph, c, p->bgrids, p->btasks[ph][c], p->bntasks[ph][c], tk, p->tabs.tw32, nb,
+        HIPCHK(batched_launch(ph, c, p->bgrids, p->btasks[ph][c], p->bntasks[ph][c], tk, p->tabs.tw32, p->tabs.stw64, nb,
                               stamp_at(p, ph == 0 ? ST_START : ST_MID), ph == 0 ? nullptr : stamp_at(p, ST_END),
                               p->stream));
     }
@@ -2709,7 +2709,7 @@ int batched_autotune(hpxfft_plan_s *p)
                     hipLaunchKernelGGL(hpxfft_dev::zero_u32_kernel<0>, dim3(1), dim3(64), 0, p->stream, tk,
                                        (long long)BATCH_QUEUES);
                     (void)hipEventRecord(a, p->stream);
-                    if (batched_launch(ph, c, p->bgrids, p->btasks[ph][c], p->bntasks[ph][c], tk, p->tabs.tw32, nb,
+                    if (batched_launch(ph, c, p->bgrids, p->btasks[ph][c], p->bntasks[ph][c], tk, p->tabs.tw32, p->tabs.stw64, nb,
                                        nullptr, nullptr, p->stream) != hipSuccess)
                         rc = fail(HPXFFT_HIP_ERROR, "batched autotune launch failed");
                     (void)hipEventRecord(b, p->stream);
@@ -2779,7 +2779,7 @@ int plan_batched(hpxfft_plan_s *p)
                 }
                 else
                 {
-                    const int w = std::max(1, pts / nx), ncols = ny / 2 + 1;
+                    const int w = batched_col_width(c, nx), ncols = ny / 2 + 1;
                     for (int st = 0; st * w < ncols; ++st, ++nt)
                     {
                         tasks.resize((size_t)(nt + 1) * tb);

@@ -20,14 +20,15 @@
 //            CFG 1: PTS 2048,  8 points/thread, 256 threads (radix 8)
 //            CFG 2: PTS 8192, 16 points/thread, 512 threads
 //            CFG 3: PTS 16384, 16 points/thread, 1024 threads
-//   columns: CFG 0: PTS 8192, 16 points/thread, 512 threads
+//   columns: CFG 0: PTS 8192, 16 points/thread, 512 threads; grids of 1024 and
+//                   2048 rows 16384 points, 32 points/thread (bcol_long)
 //            CFG 1: PTS 4096, 16 points/thread, 256 threads
 //            CFG 2: PTS 8192,  8 points/thread, 1024 threads (radix 8)
 //            CFG 3: PTS 16384, 16 points/thread, 1024 threads (a 2048-row
 //                   grid's strip is 8 columns: 64-byte row segments, not 32)
 #pragma once
 
-#include "fft_kernels.hpp"
+#include "fft_col_long.hpp"
 
 namespace hpxfft_dev {
 
@@ -56,6 +57,20 @@ template <> struct bcol_cfg<0> { static constexpr int PTS = 8192, E = 16, NT = 5
 template <> struct bcol_cfg<1> { static constexpr int PTS = 4096, E = 16, NT = 256; };
 template <> struct bcol_cfg<2> { static constexpr int PTS = 8192, E = 8, NT = 1024; };
 template <> struct bcol_cfg<3> { static constexpr int PTS = 16384, E = 16, NT = 1024; };
+
+// Column tasks of CFG 0 on grids of 1024 and 2048 rows hold 32 points per thread, as
+// the long columns do (fft_col_long.hpp): 16 and 8 columns, row segments of 128 and
+// 64 bytes, where 8192 points are 8 and 4 columns.  The segments bound those grids
+// (HBM moves 64-byte ones at 4.3 TB/s, 32-byte ones at 3.2), and real and imaginary
+// halves exchanged apart keep the workgroup's LDS, so two still share a CU.  512
+// grids of 64 .. 2048 per side: column phase 605 -> 474 us (2.7 -> 3.4 TB/s); with the
+// wide tasks on 2048 rows only, 23 us slower.
+template <int CFG, int LGX> constexpr bool bcol_long() { return CFG == 0 && LGX >= 10; }
+// adjacent columns of a task
+template <int CFG, int LGX> constexpr int bcol_width()
+{
+    return (bcol_cfg<CFG>::PTS << (bcol_long<CFG, LGX>() ? 1 : 0)) >> LGX;
+}
 
 // largest LDS footprint over the row lengths of a configuration (complex elements)
 template <int CFG> constexpr int brow_lds()
@@ -97,9 +112,18 @@ __device__ __forceinline__ int take_ticket(unsigned *ticket, int ntasks, unsigne
         *shared_slot = (unsigned)t;
     }
     __syncthreads();
-    const int t = (int)*shared_slot;
+    const int t = __builtin_amdgcn_readfirstlane((int)*shared_slot);   // uniform: task and grid in scalar registers
     __syncthreads();
     return t;
+}
+
+// the grid's pointer, known to lie in global memory: loaded from a descriptor it is
+// generic, and its loads and stores were flat ones with a 64-bit vector address each
+__device__ __forceinline__ float *grid_data(const BGrid &g)
+{
+    const unsigned long long d = reinterpret_cast<uintptr_t>(g.data);
+    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)d), hi = __builtin_amdgcn_readfirstlane((unsigned)(d >> 32));
+    return (float *)(__attribute__((address_space(1))) float *)(((unsigned long long)hi << 32) | lo);
 }
 
 // non-inlined: keeps each size's index arithmetic inside the task loop
@@ -114,11 +138,11 @@ __device__ __attribute__((noinline)) void brow_task(const BGrid &g, int row0, co
     static_assert(EN::NT == C::NT, "thread count");
     static_assert(EN::LDS_ELEMS <= brow_lds<CFG>(), "LDS");
     RowArgs a{};
-    a.in = g.data;
-    a.out = g.data;
+    a.in = a.out = grid_data(g);
     a.ld_in = 2 * (L + 1);
     a.ld_out = 2 * (L + 1);
-    a.nrows = g.nx;
+    a.nrows = __builtin_amdgcn_readfirstlane(g.nx);
+    row0 = __builtin_amdgcn_readfirstlane(row0);
     a.tw = tw32 + 2 * (2 * L);   // w_{2L} table
     row_r2c_body<float, float, float, L, C::E, NSEQ, false>(a, 0, row0, lds, nullptr);
 }
@@ -151,29 +175,56 @@ batched_rows_kernel(const BGrid *__restrict__ grids, const BTask *__restrict__ t
     stamp_first(ts, t_start);
 }
 
+// One task.  CFG 0: inlined with all others, and t made anew for each task so that no
+// index arithmetic leaves the loop: a kernel with calls spilled 57-97 VGPRs around the
+// 32-point tasks.  The other shapes stay functions.
 template <int CFG, int LGX>
-__device__ __attribute__((noinline)) void bcol_task(const BGrid &g, int strip, const float *tw32, cpx<float> *lds)
+__device__ __forceinline__ void bcol_task_body(const BGrid &g, int strip, const float *tw32, const cpx<double> *stw64,
+                                               cpx<float> *lds)
 {
     using C = bcol_cfg<CFG>;
     constexpr int N = 1 << LGX;
-    constexpr int W = C::PTS / N;
-    using EN = Engine<float, N, C::E, W, true, false>;
-    static_assert(EN::NT == C::NT, "thread count");
-    static_assert(EN::LDS_ELEMS <= bcol_lds<CFG>(), "LDS");
-    const int ncols = g.ny / 2 + 1;
+    constexpr int W = bcol_width<CFG, LGX>();
     ColArgs a{};
-    a.in = g.data;
-    a.out = g.data;
-    a.pitch = ncols;
-    a.ncols = ncols;
+    a.in = a.out = grid_data(g);
+    a.ncols = __builtin_amdgcn_readfirstlane(g.ny) / 2 + 1;
+    a.pitch = a.ncols;
+    strip = __builtin_amdgcn_readfirstlane(strip);
     a.tw_L = tw32 + 2 * N;
-    col_body<float, float, float, N, C::E, W, false, false>(a, 0, strip, lds, nullptr);
+    int t = threadIdx.x;
+    if constexpr (CFG == 0) asm volatile("" : "+v"(t));
+    if constexpr (bcol_long<CFG, LGX>())
+    {
+        using CL = collong<float, LGX, C::NT>;
+        static_assert(CL::W == W && CL::LP * W <= 2 * bcol_lds<CFG>(), "LDS");
+        a.stw64 = stw64;
+        col_long_body<CL, false>(a, 0, strip, reinterpret_cast<float *>(lds), t);
+    }
+    else
+    {
+        using EN = Engine<float, N, C::E, W, true, false>;
+        static_assert(EN::NT == C::NT, "thread count");
+        static_assert(EN::LDS_ELEMS <= bcol_lds<CFG>(), "LDS");
+        col_body<float, float, float, N, C::E, W, false, false>(a, 0, strip, lds, nullptr, t);
+    }
+}
+template <int CFG, int LGX>
+__device__ __attribute__((noinline)) void bcol_task_call(const BGrid &g, int strip, const float *tw32, cpx<float> *lds)
+{
+    bcol_task_body<CFG, LGX>(g, strip, tw32, nullptr, lds);
+}
+template <int CFG, int LGX>
+__device__ __forceinline__ void bcol_task(const BGrid &g, int strip, const float *tw32, const cpx<double> *stw64,
+                                          cpx<float> *lds)
+{
+    if constexpr (CFG == 0) bcol_task_body<CFG, LGX>(g, strip, tw32, stw64, lds);
+    else bcol_task_call<CFG, LGX>(g, strip, tw32, lds);
 }
 
 template <int CFG>
-__global__ void __launch_bounds__(bcol_cfg<CFG>::NT)
+__global__ void __launch_bounds__(bcol_cfg<CFG>::NT, 4)
 batched_cols_kernel(const BGrid *__restrict__ grids, const BTask *__restrict__ tasks, int ntasks,
-                    unsigned *ticket, const float *__restrict__ tw32, Stamps ts)
+                    unsigned *ticket, const float *__restrict__ tw32, const cpx<double> *__restrict__ stw64, Stamps ts)
 {
     const unsigned long long t_start = stamp_now(ts, ntasks);
     __shared__ cpx<float> lds[bcol_lds<CFG>()];
@@ -186,12 +237,12 @@ batched_cols_kernel(const BGrid *__restrict__ grids, const BTask *__restrict__ t
         const BGrid g = grids[task.grid];
         switch (g.lgx)
         {
-        case 6: bcol_task<CFG, 6>(g, task.first, tw32, lds); break;
-        case 7: bcol_task<CFG, 7>(g, task.first, tw32, lds); break;
-        case 8: bcol_task<CFG, 8>(g, task.first, tw32, lds); break;
-        case 9: bcol_task<CFG, 9>(g, task.first, tw32, lds); break;
-        case 10: bcol_task<CFG, 10>(g, task.first, tw32, lds); break;
-        default: bcol_task<CFG, 11>(g, task.first, tw32, lds); break;
+        case 6: bcol_task<CFG, 6>(g, task.first, tw32, stw64, lds); break;
+        case 7: bcol_task<CFG, 7>(g, task.first, tw32, stw64, lds); break;
+        case 8: bcol_task<CFG, 8>(g, task.first, tw32, stw64, lds); break;
+        case 9: bcol_task<CFG, 9>(g, task.first, tw32, stw64, lds); break;
+        case 10: bcol_task<CFG, 10>(g, task.first, tw32, stw64, lds); break;
+        default: bcol_task<CFG, 11>(g, task.first, tw32, stw64, lds); break;
         }
         __syncthreads();
     }

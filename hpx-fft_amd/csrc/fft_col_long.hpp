@@ -161,23 +161,19 @@ __device__ __forceinline__ void col_long_last(cpx<typename C::real> *v, typename
     }
 }
 
-// blockIdx.x = strip, .z = grid; from a.in to a.out in the same layout (in
-// place for the forward transform).  CONJ: the inverse, conj(DFT(conj .)).
-template <typename T, int LG, int NTH, bool CONJ>
-__global__ void __launch_bounds__(NTH, 4) col_long_kernel(ColArgs a)
+// one strip of W columns of grid b, from a.in to a.out in the same layout (in place
+// for the forward transform).  CONJ: the inverse, conj(DFT(conj .)).  Shared with the
+// batched column-phase kernel.
+template <typename C, bool CONJ>
+__device__ __forceinline__ void col_long_body(const ColArgs &a, long long b, int strip, typename C::real *lds, int t)
 {
-    using C = collong<T, LG, NTH>;
+    using T = typename C::real;
     constexpr int W = C::W, JT = C::JT, M = C::M, RL = C::RL, NSL = C::NSL, NB = C::NB;
-    __shared__ T lds[C::LP * W];
-    const unsigned long long t_start = stamp_now(a.ts, a.ncols);
-    const int t = threadIdx.x, w = t % W, jj = t / W;
-    const blk3 bk = xcd_block();   // neighbouring strips share lines: one XCD
-    const int c = bk.x * W + w;
+    const int w = t % W, jj = t / W;
+    const int c = strip * W + w;
     const bool valid = c < a.ncols;
     const int cl = valid ? c : a.ncols - 1;   // lanes past the last column load it and store nothing
-    const long long base = (long long)bk.z * a.dist + cl + (long long)jj * a.pitch;
-    const T *in = reinterpret_cast<const T *>(a.in) + 2 * base;
-    T *out = reinterpret_cast<T *>(a.out) + 2 * base;
+    const T *in = reinterpret_cast<const T *>(a.in) + 2 * (b * a.dist + cl + (long long)jj * a.pitch);
     cpx<T> v[16 * NB];
 #pragma unroll
     for (int u = 0; u < 16 * NB; ++u)
@@ -188,6 +184,11 @@ __global__ void __launch_bounds__(NTH, 4) col_long_kernel(ColArgs a)
     col_long_stages<C, 0>(v, lds, reinterpret_cast<const cpx<double> *>(a.stw64), jj, w);
     if constexpr (RL > 1) col_long_last<C>(v, lds, reinterpret_cast<const cpx<T> *>(a.tw_L), jj, w);
     if (!valid) return;
+    // the stores' addresses are formed after the stages (in place they are the loads',
+    // which the batched kernel else kept, spilled)
+    int js = jj;
+    asm volatile("" : "+v"(js));
+    T *out = reinterpret_cast<T *>(a.out) + 2 * (b * a.dist + cl + (long long)js * a.pitch);
     constexpr int R = RL > 1 ? RL : 16, STR = RL > 1 ? NSL : M;
 #pragma unroll
     for (int u = 0; u < 16 * NB; ++u)
@@ -195,6 +196,17 @@ __global__ void __launch_bounds__(NTH, 4) col_long_kernel(ColArgs a)
         const cpx<T> z = v[u];
         stor<T>::st(out + 2 * a.pitch * ((u / R) * JT + (u % R) * STR), CONJ ? conjc(z) : z);
     }
+}
+
+// blockIdx.x = strip, .z = grid
+template <typename T, int LG, int NTH, bool CONJ>
+__global__ void __launch_bounds__(NTH, 4) col_long_kernel(ColArgs a)
+{
+    using C = collong<T, LG, NTH>;
+    __shared__ T lds[C::LP * C::W];
+    const unsigned long long t_start = stamp_now(a.ts, a.ncols);
+    const blk3 bk = xcd_block();   // neighbouring strips share lines: one XCD
+    col_long_body<C, CONJ>(a, bk.z, bk.x, lds, threadIdx.x);
     stamp(a.ts, t_start);
 }
 

@@ -301,11 +301,10 @@ row_r2c_kernel(RowArgs a)
 // from its exact maximum, written to out_exp.
 template <typename T, typename SI, typename SO, int L, int E, int W, bool SPLIT, bool CONJ>
 __device__ __forceinline__ void col_body(const ColArgs &a, long long b, int strip,
-                                         typename Engine<T, L, E, W, true, SPLIT>::lds_t *lds, unsigned *smax)
+                                         typename Engine<T, L, E, W, true, SPLIT>::lds_t *lds, unsigned *smax, int t)
 {
     using EN = Engine<T, L, E, W, true, SPLIT>;
     constexpr bool OUT16 = is16<SO>();
-    const int t = threadIdx.x;
     const int col0 = strip * W;
     const int nvalid = min(W, a.ncols - col0);
     const SI *in = reinterpret_cast<const SI *>(a.in) + 2 * b * a.dist;   // dist counts complex elements
@@ -401,7 +400,7 @@ col_kernel(ColArgs a)
     __shared__ unsigned smax[is16<S>() ? W : 1];
     const unsigned long long t_start = stamp_now(a.ts, a.ncols);
     const blk3 bk = xcd_block();
-    col_body<T, S, S, L, E, W, SPLIT, CONJ>(a, bk.z, bk.x, lds, smax);
+    col_body<T, S, S, L, E, W, SPLIT, CONJ>(a, bk.z, bk.x, lds, smax, threadIdx.x);
     stamp(a.ts, t_start);
 }
 

@@ -15,6 +15,13 @@ int batched_pts(int phase, int cfg)
     return cfg == 0 ? bcol_cfg<0>::PTS : cfg == 1 ? bcol_cfg<1>::PTS : cfg == 2 ? bcol_cfg<2>::PTS : bcol_cfg<3>::PTS;
 }
 
+int batched_col_width(int cfg, int nx)
+{
+    const bool wide = cfg == 0 && nx >= 1 << 10;   // bcol_long
+    static_assert(bcol_width<0, 10>() == 16 && bcol_width<0, 11>() == 8 && bcol_width<0, 9>() == 16, "task widths");
+    return (batched_pts(1, cfg) << (wide ? 1 : 0)) / nx;
+}
+
 static int nthreads(int phase, int cfg)
 {
     if (phase == 0)
@@ -48,9 +55,10 @@ int batched_resident_blocks(int phase, int cfg)
 }
 
 hipError_t batched_launch(int phase, int cfg, const void *grids, const void *tasks, int ntasks, unsigned *ticket,
-                          const float *tw32, int nblocks, unsigned long long *begin, unsigned long long *end, hipStream_t s)
+                          const float *tw32, const void *stw64, int nblocks, unsigned long long *begin, unsigned long long *end, hipStream_t s)
 {
     const Stamps ts{begin, end};
+    const cpx<double> *st = reinterpret_cast<const cpx<double> *>(stw64);
     const BGrid *g = reinterpret_cast<const BGrid *>(grids);
     const BTask *t = reinterpret_cast<const BTask *>(tasks);
     const dim3 grid((unsigned)nblocks), block((unsigned)nthreads(phase, cfg));
@@ -63,10 +71,10 @@ hipError_t batched_launch(int phase, int cfg, const void *grids, const void *tas
     }
     else
     {
-        if (cfg == 0) hipLaunchKernelGGL(batched_cols_kernel<0>, grid, block, 0, s, g, t, ntasks, ticket, tw32, ts);
-        else if (cfg == 1) hipLaunchKernelGGL(batched_cols_kernel<1>, grid, block, 0, s, g, t, ntasks, ticket, tw32, ts);
-        else if (cfg == 2) hipLaunchKernelGGL(batched_cols_kernel<2>, grid, block, 0, s, g, t, ntasks, ticket, tw32, ts);
-        else hipLaunchKernelGGL(batched_cols_kernel<3>, grid, block, 0, s, g, t, ntasks, ticket, tw32, ts);
+        if (cfg == 0) hipLaunchKernelGGL(batched_cols_kernel<0>, grid, block, 0, s, g, t, ntasks, ticket, tw32, st, ts);
+        else if (cfg == 1) hipLaunchKernelGGL(batched_cols_kernel<1>, grid, block, 0, s, g, t, ntasks, ticket, tw32, st, ts);
+        else if (cfg == 2) hipLaunchKernelGGL(batched_cols_kernel<2>, grid, block, 0, s, g, t, ntasks, ticket, tw32, st, ts);
+        else hipLaunchKernelGGL(batched_cols_kernel<3>, grid, block, 0, s, g, t, ntasks, ticket, tw32, st, ts);
     }
     return hipGetLastError();
 }
