@@ -555,6 +555,14 @@ template <typename T, int LG> constexpr int c2r_min_waves()
     return sizeof(T) == 8 && LG == 13 ? 4 : big_min_waves<T, LG>();
 }
 
+// Rows whose exchanges are split form Z in registers, from G[k], G[L-k] and the
+// twiddle of each of the thread's own points: through LDS they built one component per
+// pass, reading G twice all the same, with 4 barriers more.  FP64 2048 x 32768 c2r 766
+// -> 719 us, 2048 x 16384 321 -> 314, 256 x 16384 38.7 -> 36.1; FP32 2048 x 32768 383 ->
+// 353.  FP32 rows of 2^13 points keep the LDS form (2048 x 16384 189 against 198), and so
+// do rows of 2^11, which read G once through it (16 x 4096^2 FP32 backward 120 us less).
+template <typename T, int LG> constexpr bool c2r_direct() { return LG == 14 || (LG == 13 && sizeof(T) == 8); }
+
 template <typename T, typename S, int LG, bool HALVE>
 __global__ void __launch_bounds__((1 << LG) / (16 * big_nb<T, LG>()), (c2r_min_waves<T, LG>()))
 row_c2r_big_kernel(RowArgs a)
@@ -577,39 +585,21 @@ row_c2r_big_kernel(RowArgs a)
     const cpx<T> *tw = reinterpret_cast<const cpx<T> *>(a.tw);
     const cpx<double> *stw64 = reinterpret_cast<const cpx<double> *>(a.stw64);
 
-    // pair tasks in chunks of CH: each chunk's loads of G[k], G[L-k] and the
-    // twiddle are issued together (tasks past L/2 read the pair L/2 and write
-    // nothing); split rows build one component per pass, reading G again
-    constexpr int CH = 4;
-    auto pair = [&](int k, const cpx<T> &g0, const cpx<T> &g1, const cpx<T> &w, cpx<T> &z0, cpx<T> &z1) {
-        if (k == 0)
-        {
-            // H0 = Re G0, HL = Re GL: Z0 = (H0 + HL) + i (H0 - HL)
-            z0 = conjc(cpx<T>{g0.x + g1.x, g0.x - g1.x});
-            z1 = z0;
-        }
-        else
-        {
-            const T hs = HALVE ? T(0.5) : T(1);
-            const cpx<T> h0 = scal(g0, hs), h1 = scal(g1, hs);
-            const cpx<T> s0 = h0 + conjc(h1), d0 = cmul(h0 - conjc(h1), conjc(w));
-            const cpx<T> s1 = h1 + conjc(h0), d1 = cmul(h1 - conjc(h0), cpx<T>{-w.x, -w.y});   // conj w^{L-k} = -w^k
-            z0 = conjc(cpx<T>{s0.x - d0.y, s0.y + d0.x});
-            z1 = conjc(cpx<T>{s1.x - d1.y, s1.y + d1.x});
-        }
-    };
     cpx<T> v[16 * NB];
-#pragma unroll
-    for (int h = 0; h < (B::SPLIT ? 2 : 1); ++h)
+    if constexpr (c2r_direct<T, LG>())
     {
-#pragma unroll 1
-        for (int c0 = 0; c0 < NTASK; c0 += CH)
+        // each thread's stage-0 inputs v[16 b + r] = conj Z[k], k = t + b NT + r M, formed in
+        // registers from G[k], G[L-k] and w_{2L}^k (exact for every k < L), CH at a time
+        constexpr int CH = 4;
+        const T hs = HALVE ? T(0.5) : T(1);
+#pragma unroll
+        for (int c0 = 0; c0 < 16 * NB; c0 += CH)
         {
             cpx<T> G0[CH], G1[CH], W[CH];
 #pragma unroll
             for (int i = 0; i < CH; ++i)
             {
-                const int k = min(t + (c0 + i) * NT, L / 2);
+                const int k = t + ((c0 + i) / 16) * NT + ((c0 + i) % 16) * M;
                 G0[i] = stor<S>::ld(irow + 2 * k);
                 G1[i] = stor<S>::ld(irow + 2 * (L - k));
                 W[i] = tw[k];
@@ -617,34 +607,85 @@ row_c2r_big_kernel(RowArgs a)
 #pragma unroll
             for (int i = 0; i < CH; ++i)
             {
-                const int k = t + (c0 + i) * NT;
-                if (c0 + i >= NTASK || k > L / 2) continue;
-                cpx<T> z0, z1;
-                pair(k, G0[i], G1[i], W[i], z0, z1);
-                if constexpr (!B::SPLIT)
+                const cpx<T> h0 = scal(G0[i], hs), h1 = scal(G1[i], hs);
+                const cpx<T> s0 = h0 + conjc(h1), d0 = cmul(h0 - conjc(h1), conjc(W[i]));
+                v[c0 + i] = conjc(cpx<T>{s0.x - d0.y, s0.y + d0.x});
+            }
+            // H0 = Re G0, HL = Re GL: Z0 = (H0 + HL) + i (H0 - HL)
+            if (c0 == 0 && t == 0) v[0] = conjc(cpx<T>{G0[0].x + G1[0].x, G0[0].x - G1[0].x});
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    else
+    {
+        // pair tasks in chunks of CH: each chunk's loads of G[k], G[L-k] and the
+        // twiddle are issued together (tasks past L/2 read the pair L/2 and write
+        // nothing); split rows build one component per pass, reading G again
+        constexpr int CH = 4;
+        auto pair = [&](int k, const cpx<T> &g0, const cpx<T> &g1, const cpx<T> &w, cpx<T> &z0, cpx<T> &z1) {
+            if (k == 0)
+            {
+                // H0 = Re G0, HL = Re GL: Z0 = (H0 + HL) + i (H0 - HL)
+                z0 = conjc(cpx<T>{g0.x + g1.x, g0.x - g1.x});
+                z1 = z0;
+            }
+            else
+            {
+                const T hs = HALVE ? T(0.5) : T(1);
+                const cpx<T> h0 = scal(g0, hs), h1 = scal(g1, hs);
+                const cpx<T> s0 = h0 + conjc(h1), d0 = cmul(h0 - conjc(h1), conjc(w));
+                const cpx<T> s1 = h1 + conjc(h0), d1 = cmul(h1 - conjc(h0), cpx<T>{-w.x, -w.y});   // conj w^{L-k} = -w^k
+                z0 = conjc(cpx<T>{s0.x - d0.y, s0.y + d0.x});
+                z1 = conjc(cpx<T>{s1.x - d1.y, s1.y + d1.x});
+            }
+        };
+#pragma unroll
+        for (int h = 0; h < (B::SPLIT ? 2 : 1); ++h)
+        {
+#pragma unroll 1
+            for (int c0 = 0; c0 < NTASK; c0 += CH)
+            {
+                cpx<T> G0[CH], G1[CH], W[CH];
+#pragma unroll
+                for (int i = 0; i < CH; ++i)
                 {
-                    cpx<T> *l = reinterpret_cast<cpx<T> *>(lds);
-                    l[B::pad(k)] = z0;
-                    if (k != 0) l[B::pad(L - k)] = z1;
+                    const int k = min(t + (c0 + i) * NT, L / 2);
+                    G0[i] = stor<S>::ld(irow + 2 * k);
+                    G1[i] = stor<S>::ld(irow + 2 * (L - k));
+                    W[i] = tw[k];
                 }
-                else
+#pragma unroll
+                for (int i = 0; i < CH; ++i)
                 {
-                    lds[B::pad(k)] = h ? z0.y : z0.x;
-                    if (k != 0) lds[B::pad(L - k)] = h ? z1.y : z1.x;
+                    const int k = t + (c0 + i) * NT;
+                    if (c0 + i >= NTASK || k > L / 2) continue;
+                    cpx<T> z0, z1;
+                    pair(k, G0[i], G1[i], W[i], z0, z1);
+                    if constexpr (!B::SPLIT)
+                    {
+                        cpx<T> *l = reinterpret_cast<cpx<T> *>(lds);
+                        l[B::pad(k)] = z0;
+                        if (k != 0) l[B::pad(L - k)] = z1;
+                    }
+                    else
+                    {
+                        lds[B::pad(k)] = h ? z0.y : z0.x;
+                        if (k != 0) lds[B::pad(L - k)] = h ? z1.y : z1.x;
+                    }
                 }
             }
-        }
-        __syncthreads();
-        // each thread's stage-0 inputs v[16 b + r] = z[t + b NT + r M]
+            __syncthreads();
+            // each thread's stage-0 inputs v[16 b + r] = z[t + b NT + r M]
 #pragma unroll
-        for (int u = 0; u < 16 * NB; ++u)
-        {
-            const int e = B::pad(t + (u / 16) * NT + (u % 16) * M);
-            if constexpr (!B::SPLIT) v[u] = reinterpret_cast<const cpx<T> *>(lds)[e];
-            else if (h) v[u].y = lds[e];
-            else v[u].x = lds[e];
+            for (int u = 0; u < 16 * NB; ++u)
+            {
+                const int e = B::pad(t + (u / 16) * NT + (u % 16) * M);
+                if constexpr (!B::SPLIT) v[u] = reinterpret_cast<const cpx<T> *>(lds)[e];
+                else if (h) v[u].y = lds[e];
+                else v[u].x = lds[e];
+            }
+            __syncthreads();
         }
-        __syncthreads();
     }
     radix16_stages<T, L, NB, 0>(v, lds, stw64, t);
     constexpr int NS = B::ns(B::NR16 - 1);
