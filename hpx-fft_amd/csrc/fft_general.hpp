@@ -150,13 +150,14 @@ template <typename T, int R> __device__ __forceinline__ void dft_small(cpx<T> *x
 }
 
 // butterflies of a register stage that a thread takes per iteration.  Two keep more
-// loads in flight; where two FP64 butterflies of radix 7 or 8, or any two in the
-// 1024-thread build, need more than the 128 VGPRs of 4 waves per SIMD, one: with two,
-// 40-50 VGPRs were spilled (2310 x 2310 x 4 FP64 582 -> 507 us, 3000 x 3000 108 ->
-// 100, 9000 x 18000 4570 -> 4000).
-template <typename T, int R, int NTMAX> constexpr int gen_unroll()
+// loads in flight; two of radix 7 or 8, and any two in the 1024-thread build, need
+// more than the 128 VGPRs of 4 waves per SIMD (FP64 spilled 40-50), so those go one by
+// one: 2310 x 2310 x 4 FP64 582 -> 507 us, 3000 x 3000 108 -> 100, 9000 x 18000 4570
+// -> 4000, FP32 7000 x 14000 1200 -> 1060.  One for all radices was slower (9000 x
+// 18000 4370).
+template <int R, int NTMAX> constexpr int gen_unroll()
 {
-    return sizeof(T) == 8 && (R >= 7 || NTMAX != GEN_NT) ? 1 : 2;
+    return R >= 7 || NTMAX != GEN_NT ? 1 : 2;
 }
 
 // one Stockham stage of radix R (2, 3, 4, 5, 7, 8) over nseq sequences, A -> B
@@ -167,7 +168,7 @@ __device__ void gen_stage_reg(const cpx<T> *A, cpx<T> *B, int nseq, int n, int N
     const float inv_m = 1.0f / (float)m, inv_ns = 1.0f / (float)Ns;
     // UN butterflies per iteration (independent loads in flight together);
     // twiddles w^{qk} as powers of the one table value w^k, in FP64
-    constexpr int UN = gen_unroll<T, R, NTMAX>();
+    constexpr int UN = gen_unroll<R, NTMAX>();
     const int NTH = gen_nth<NTMAX>();
     for (int b0 = t; b0 < nb; b0 += UN * NTH)
     {
@@ -223,7 +224,7 @@ __device__ void gen_stage_ip(cpx<T> *A, int nseq, int n, int Ls, const cpx<doubl
 {
     const int t = threadIdx.x, m = n / R, nb = nseq * m, tstep = n / (R * Ls);
     const float inv_m = 1.0f / (float)m, inv_ls = 1.0f / (float)Ls;
-    constexpr int UN = gen_unroll<T, R, NTMAX>();
+    constexpr int UN = gen_unroll<R, NTMAX>();
     const int NTH = gen_nth<NTMAX>();
     for (int b0 = t; b0 < nb; b0 += UN * NTH)
     {
@@ -381,7 +382,7 @@ __device__ void gen_stage_dif(cpx<T> *A, int nseq, int n, int Lb, const cpx<doub
 {
     const int t = threadIdx.x, per = n / R, nb = nseq * per, m = Lb / R, tstep = n / Lb;
     const float inv_per = 1.0f / (float)per, inv_m = 1.0f / (float)m;
-    constexpr int UN = gen_unroll<T, R, NTMAX>();
+    constexpr int UN = gen_unroll<R, NTMAX>();
     const int NTH = gen_nth<NTMAX>();
     for (int b0 = t; b0 < nb; b0 += UN * NTH)
     {
