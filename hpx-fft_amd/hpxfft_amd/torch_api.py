@@ -39,8 +39,9 @@ def planning_effort() -> str:
 
 
 def _get_plan(nx: int, ny: int, batch: int, precision: str, ld_in: int, ld_out: int, device: torch.device) -> Plan:
-    stream = torch.cuda.current_stream(device)
-    key = (nx, ny, batch, precision, ld_in, ld_out, device.index, stream.cuda_stream, _effort)
+    # the handle alone: the Stream object took 1.9 of the 12.5 us of a small call
+    stream = torch._C._cuda_getCurrentRawStream(device.index)
+    key = (nx, ny, batch, precision, ld_in, ld_out, device.index, stream, _effort)
     p = _plans.get(key)
     if p is None:
         with torch.cuda.device(device):
