@@ -14,9 +14,9 @@
 // stage, so the product with Bh takes no exchange: 4 exchanges in all for 4096
 // points (6 where L is no power of 16).  len <= L/2, so the first stage's upper
 // inputs are zero, and its upper outputs are never formed.
-// In-LDS form -> this one (us, whole transform): FP64 2039 x 4078 206 -> 125, 1021 x
-// 1024 48 -> 28, 1024 x 8186 168 -> 102, 67 x 1024 30 -> 14; FP32 2039 x 1024 58 -> 33,
-// 8191 x 1024 190 -> 164 (the small grids' figures hold about 10 us of phase events
+// In-LDS form -> this one (us, whole transform): FP64 2039 x 4078 206 -> 106, 1021 x
+// 1024 48 -> 28, 1024 x 8186 168 -> 95, 67 x 1024 30 -> 14; FP32 2039 x 1024 58 -> 34,
+// 8191 x 1024 190 -> 141 (the small grids' figures hold about 10 us of phase events
 // that the in-LDS side still recorded).
 #pragma once
 
@@ -56,11 +56,12 @@ template <typename T, int LG, bool COL> struct bluecfg
         constexpr int R = RL > 1 ? RL : 16, STR = RL > 1 ? NSL : M;
         return jj + (u / R) * JT + (u % R) * STR;
     }
-    // waves per SIMD that the registers are cut to: 2 (up to 256 VGPRs, no spills).  At
-    // 4 (128) every FP64 form spills 30-50 VGPRs: FP64 1021 x 1024 34.7 against
-    // 27.8 us, 1024 x 4078 57.0 against 50.0.  FP64 rows of 2^13 points keep 4,
-    // two 512-thread workgroups per CU instead of one: 1024 x 8186 102 against 119
-    static constexpr int WAVES = sizeof(T) == 8 && !COL && LG == 13 ? 4 : 2;
+    // waves per SIMD that the registers are cut to: 4 (128 VGPRs, no spills), which
+    // lets two 512-thread workgroups share a CU (FP64 2039 x 1024 at 2: 51 us, at 4:
+    // 43).  Two FP32 butterflies per thread spill 20 VGPRs there and take 2 (2039 x 1024
+    // 38.4 -> 34.7), but rows of 2^14 points still gain by two workgroups (1024 x 16382
+    // 171 -> 138)
+    static constexpr int WAVES = NB == 2 && LG < 14 ? 2 : 4;
     static_assert(W >= 1 && JT * NB == M, "threads cover the butterflies");
 };
 
@@ -124,6 +125,11 @@ __device__ __forceinline__ void blue_fft(cpx<typename C::real> *v, typename C::r
     asm volatile("" : "+v"(jj));
     col_long_stages<C, 0>(v, lds, g.stw64, jj, w);
     if constexpr (C::RL > 1) col_long_last<C>(v, lds, tw, jj, w);
+    // the outputs are formed here: else the last stage sinks into the callers' guarded
+    // stores, below the chirp's loads
+#pragma unroll
+    for (int u = 0; u < 16 * C::NB; ++u)
+        if (C::out_e(u, 0) < C::L / 2) asm volatile("" : "+v"(v[u].x), "+v"(v[u].y));
 #pragma unroll
     for (int u = 0; u < 16 * C::NB; ++u)
     {
