@@ -183,6 +183,13 @@ __device__ __forceinline__ void col_long_body(const ColArgs &a, long long b, int
     }
     col_long_stages<C, 0>(v, lds, reinterpret_cast<const cpx<double> *>(a.stw64), jj, w);
     if constexpr (RL > 1) col_long_last<C>(v, lds, reinterpret_cast<const cpx<T> *>(a.tw_L), jj, w);
+    // FP64: the outputs are formed here, before the guard (the last stage else sinks
+    // below it): 4096 x 2048 77.0 -> 73.8 us, 16 x 2048^2 530 -> 520; FP32 4096^2 lost 1%
+    if constexpr (sizeof(T) == 8)
+    {
+#pragma unroll
+        for (int u = 0; u < 16 * NB; ++u) asm volatile("" : "+v"(v[u].x), "+v"(v[u].y));
+    }
     if (!valid) return;
     // the stores' addresses are formed after the stages (in place they are the loads',
     // which the batched kernel else kept, spilled)
