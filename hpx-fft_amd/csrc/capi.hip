@@ -321,6 +321,11 @@ struct hpxfft_plan_s
     bool own_ends = true;        // false: the exec is the middle of a longer one, which stamps start and end itself
     double clock_hz = 1e8;
     bool ran = false;
+    // the host entry point reads its run's times once, when it has waited for it
+    // anyway (three reads by get_measurement: 30 us); not on a plan with captured
+    // execs, whose replays stamp newer ones unseen
+    bool captured = false, host_times_ok = false;
+    double host_times[5] = {};
     bool col_split = false;      // the last run's column pass was a four-step
     bool col_first = false;      // the last run was backward: the column pass before the rows
     double h2d = 0.0, d2h = 0.0;
@@ -987,10 +992,25 @@ int alloc_events(hpxfft_plan_s *p)
     return HPXFFT_OK;
 }
 
+// at the start of an exec (the null stream cannot be captured)
+void note_exec(hpxfft_plan_s *p)
+{
+    p->host_times_ok = false;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (p->stream && hipStreamIsCapturing(p->stream, &st) == hipSuccess && st != hipStreamCaptureStatusNone)
+        p->captured = true;
+}
+
 // seconds of the last exec's phases, once it has finished
 struct phase_times { double total, first, second, split_a, split_b; };
 int read_times(hpxfft_plan_s *p, phase_times &t)
 {
+    if (p->host_times_ok)
+    {
+        const double *h = p->host_times;
+        t = {h[0], h[1], h[2], h[3], h[4]};
+        return HPXFFT_OK;
+    }
     std::vector<unsigned long long> w(ST_WORDS);
     HIPCHK(hipMemcpyAsync(w.data(), p->stamps, sizeof(w[0]) * ST_WORDS, hipMemcpyDeviceToHost, p->stream));
     HIPCHK(hipStreamSynchronize(p->stream));
@@ -1536,6 +1556,7 @@ int exec_forward(hpxfft_plan_s *p, const void *d_in, void *d_out, const int *in_
     if (s16 && !col_exp) col_exp = p->col_exp_own;
     if (p->wide16) return exec_wide16(p, d_in, d_out, in_exp, col_exp);
     device_guard g(p->device);
+    note_exec(p);
     RowArgs r{};
     r.ts.begin = stamp_start(p);
     r.in = d_in;
@@ -2442,6 +2463,14 @@ int hpxfft_exec_r2c_2d_host(hpxfft_plan plan, double *inout)
         HIPCHK(hipEventSynchronize(e1.ev));
         plan->h2d = elapsed(e0.ev, in_done.ev);
         plan->d2h = elapsed(out_start.ev, e1.ev);
+        if (!plan->captured)
+        {
+            phase_times t{};
+            if (int rc = read_times(plan, t)) return rc;
+            const double h[5] = {t.total, t.first, t.second, t.split_a, t.split_b};
+            std::copy(h, h + 5, plan->host_times);
+            plan->host_times_ok = true;
+        }
         return HPXFFT_OK;
     });
 }
@@ -2461,6 +2490,7 @@ int exec_backward(hpxfft_plan_s *plan, const void *d_spec, void *d_real, bool ha
     if (plan->prec != P_F64 && plan->prec != P_F32)
         return fail(HPXFFT_INVALID_ARG, std::string(what) + " is implemented for F64 and F32 plans");
     device_guard g(plan->device);
+    note_exec(plan);
     const size_t sb = storage_bytes(plan->prec);
     const size_t bytes = plan->batch * plan->dist_out * 2 * sb;
     if (!plan->adj_work)
