@@ -895,7 +895,8 @@ std::string describe(const hpxfft_plan_s *p)
                << "exchange in re/im halves; the four-step it replaces:\n";
         }
         os << "  column c2c four-step Nx = P*Q = " << (1 << p->lgP) << " * " << (1 << p->lgQ) << " (scratch "
-           << p->scratch_bytes << " B, one block per strip)\n";
+           << p->scratch_bytes << " B, one block per strip" << (p->col_long ? "; allocated when a split is set" : "")
+           << ")\n";
         os << "    phase A: " << (1 << p->lgQ) << "-point DFTs over rows m1+P*m2, twiddle w_Nx^(m1 k2), tiles of "
            << ga.nseq << " columns, " << ga.nt << " threads\n";
         os << "    phase B: " << (1 << p->lgP) << "-point DFTs, to rows Q*k1+k2, tiles of " << gb.nseq << " columns, "
@@ -1678,9 +1679,18 @@ void split_range(int lgx, int &lo, int &hi)
     hi = std::min(COL_TILE_MAX_LG, lgx - COL_TILE_MIN_LG);
 }
 
+// the four-step scratch, on the device (current); the one-launch columns go
+// without, until a split is timed or set
+int need_scratch(hpxfft_plan_s *p)
+{
+    if (!p->scratch) HIPCHK(hipMalloc(&p->scratch, p->scratch_bytes));
+    return HPXFFT_OK;
+}
+
 // effort >= measure: time the column pass of every valid split on a zeroed
 // spectrum of the plan's shape (forward, in place) and keep the fastest.
-// If the temporary spectrum cannot be allocated the default split stays.
+// If the temporary spectrum, or the scratch of a plan whose columns are one
+// launch, cannot be allocated the default stays.
 int tune_split(hpxfft_plan_s *p)
 {
     if (int rc = alloc_events(p)) return rc;
@@ -1692,6 +1702,12 @@ int tune_split(hpxfft_plan_s *p)
     if (hipMalloc(&tmp, bytes) != hipSuccess)
     {
         (void)hipGetLastError();
+        return HPXFFT_OK;
+    }
+    if (p->col_long && need_scratch(p) != HPXFFT_OK)
+    {
+        (void)hipGetLastError();
+        (void)hipFree(tmp);
         return HPXFFT_OK;
     }
     const bool s16 = p->prec == P_F16 || p->prec == P_BF16;
@@ -1735,6 +1751,11 @@ int tune_split(hpxfft_plan_s *p)
     p->lgP = best;
     p->lgQ = p->lgx - best;
     p->col_long = best_long;
+    if (best_long)
+    {
+        (void)hipFree(p->scratch);
+        p->scratch = nullptr;
+    }
     if (rc != HPXFFT_OK) return rc;
     HIPCHK(e);
     return HPXFFT_OK;
@@ -2188,7 +2209,8 @@ int plan_common(hpxfft_plan_s *p)
         if (p->g2c.avail) HIPCHK(hipMalloc(&p->gscr, p->batch * p->g2c.points() * p->ncols * cb));
     }
     if (int rc = choose_columns(p)) return rc;
-    if (p->four_step) HIPCHK(hipMalloc(&p->scratch, p->scratch_bytes));
+    if (p->four_step && !p->col_long)
+        if (int rc = need_scratch(p)) return rc;
     if (p->prec == P_F16 || p->prec == P_BF16)
     {
         HIPCHK(hipMalloc(&p->mid_exp, sizeof(int) * p->nx * p->batch));
@@ -2901,6 +2923,8 @@ int hpxfft_plan_set_column_split(hpxfft_plan plan, int log2_p)
                                             std::to_string(hi) + "] for Nx = " + std::to_string(plan->nx));
     // the scratch holds TW-column strips of Nx rows whatever the split, and the
     // 16-bit column maxima were sized for the largest P of the range
+    device_guard g(plan->device);
+    if (int rc = need_scratch(plan)) return rc;
     plan->col_long = false;
     plan->lgP = log2_p;
     plan->lgQ = plan->lgx - log2_p;
