@@ -317,7 +317,6 @@ struct hpxfft_plan_s
     // the first launch's start, [ST_MID] the second pass's, [ST_SPLIT] the
     // four-step phase B's, then STAMP_SLOTS ends of the last launch's workgroups
     unsigned long long *stamps = nullptr;   // null: untimed (the allocation-free entry point)
-    int stamp_set = -1;          // index in the device's pool of sets (alloc_timing); -1: an allocation
     bool own_ends = true;        // false: the exec is the middle of a longer one, which stamps start and end itself
     double clock_hz = 1e8;
     bool ran = false;
@@ -940,16 +939,50 @@ double elapsed(hipEvent_t a, hipEvent_t b)
     return (double)ms * 1e-3;
 }
 
-// Stamp words for the plans of a device: STAMP_POOL sets in a static array (one
-// copy per device, zero from the start), handed out under a lock and given back
-// by free_plan; a further plan allocates its own.  A set's old values need no
-// clearing: the start words are rewritten by every exec, and earlier ends never
-// exceed later ones.  (hipMalloc and a clearing copy took 30 us per plan.)
+// Stamp words for the plans of a device: sets of ST_WORDS in blocks of STAMP_POOL
+// (1 MiB, allocated when no set is free: 64 plans per hipMalloc, which with its
+// clearing took 30 us per plan), handed out under a lock and taken back by free_plan.
+// A set's old values need no clearing: the start words are rewritten by every exec,
+// and earlier ends never exceed later ones.  Blocks stay until the process ends, and
+// the set of a plan with captured execs is handed out again only when no other is
+// free: a graph that outlives its plan stamps it at every replay.
 constexpr int STAMP_POOL = 64;
-static __device__ unsigned long long stamp_pool[STAMP_POOL][ST_WORDS];
+struct stamp_sets
+{
+    std::vector<unsigned long long *> free, worn;   // worn: stamped by graphs, oldest first
+};
 std::mutex g_stamp_mu;
-struct stamp_sets { unsigned long long *base = nullptr; uint64_t used = 0; };
 std::map<int, stamp_sets> g_stamps;
+
+// lets this thread allocate while a stream is being captured (a plan made inside a
+// capture needs no other allocation where its tables are up and it has no scratch)
+struct relaxed_capture
+{
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    bool ok = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    ~relaxed_capture()
+    {
+        if (ok) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    }
+};
+
+// another block of sets, zeroed on a stream of its own (the plan's may be captured)
+int grow_stamps(stamp_sets &d)
+{
+    relaxed_capture relaxed;
+    const size_t bytes = sizeof(unsigned long long) * ST_WORDS * STAMP_POOL;
+    unsigned long long *block = nullptr;
+    hipStream_t s = nullptr;
+    HIPCHK(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
+    hipError_t e = hipMalloc(reinterpret_cast<void **>(&block), bytes);
+    if (e == hipSuccess) e = hipMemsetAsync(block, 0, bytes, s);
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    (void)hipStreamDestroy(s);
+    if (e != hipSuccess) (void)hipFree(block);
+    HIPCHK(e);
+    for (int i = STAMP_POOL - 1; i >= 0; --i) d.free.push_back(block + (size_t)i * ST_WORDS);
+    return HPXFFT_OK;
+}
 
 // a set of stamp words for a new plan on its device (current)
 int alloc_timing(hpxfft_plan_s *p)
@@ -957,32 +990,28 @@ int alloc_timing(hpxfft_plan_s *p)
     int khz = 0;
     HIPCHK(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, p->device));
     if (khz > 0) p->clock_hz = 1e3 * khz;
+    std::lock_guard<std::mutex> lk(g_stamp_mu);
+    stamp_sets &d = g_stamps[p->device];
+    if (d.free.empty() && d.worn.empty())
+        if (int rc = grow_stamps(d)) return rc;
+    if (!d.free.empty())
     {
-        std::lock_guard<std::mutex> lk(g_stamp_mu);
-        stamp_sets &d = g_stamps[p->device];
-        if (!d.base) HIPCHK(hipGetSymbolAddress(reinterpret_cast<void **>(&d.base), HIP_SYMBOL(stamp_pool)));
-        for (int i = 0; i < STAMP_POOL; ++i)
-            if (!(d.used >> i & 1))
-            {
-                d.used |= uint64_t(1) << i;
-                p->stamp_set = i;
-                p->stamps = d.base + (size_t)i * ST_WORDS;
-                return HPXFFT_OK;
-            }
+        p->stamps = d.free.back();
+        d.free.pop_back();
     }
-    HIPCHK(hipMalloc(&p->stamps, sizeof(unsigned long long) * ST_WORDS));
-    const std::vector<unsigned long long> zero(ST_WORDS, 0);
-    HIPCHK(hipMemcpy(p->stamps, zero.data(), sizeof(zero[0]) * ST_WORDS, hipMemcpyHostToDevice));
+    else
+    {
+        p->stamps = d.worn.front();
+        d.worn.erase(d.worn.begin());
+    }
     return HPXFFT_OK;
 }
 void free_timing(hpxfft_plan_s *p)
 {
-    if (p->stamp_set >= 0)
-    {
-        std::lock_guard<std::mutex> lk(g_stamp_mu);
-        g_stamps[p->device].used &= ~(uint64_t(1) << p->stamp_set);
-    }
-    else (void)hipFree(p->stamps);
+    if (!p->stamps) return;
+    std::lock_guard<std::mutex> lk(g_stamp_mu);
+    stamp_sets &d = g_stamps[p->device];
+    (p->captured ? d.worn : d.free).push_back(p->stamps);
 }
 
 // the planning searches' events
@@ -1555,9 +1584,9 @@ int exec_forward(hpxfft_plan_s *p, const void *d_in, void *d_out, const int *in_
         return fail(HPXFFT_INVALID_ARG, "in-place exec needs ld_in == 2*ld_out and dist_in == 2*dist_out");
     const bool s16 = p->prec == P_F16 || p->prec == P_BF16;
     if (s16 && !col_exp) col_exp = p->col_exp_own;
+    note_exec(p);
     if (p->wide16) return exec_wide16(p, d_in, d_out, in_exp, col_exp);
     device_guard g(p->device);
-    note_exec(p);
     RowArgs r{};
     r.ts.begin = stamp_start(p);
     r.in = d_in;
@@ -2950,6 +2979,7 @@ int hpxfft_exec_r2c_2d_batched(hpxfft_plan plan, void *const *d_grids)
         if (!d_grids) return fail(HPXFFT_INVALID_ARG, "null grid pointer array");
         device_guard g(plan->device);
         if (int rc = batched_upload_grids(plan, d_grids)) return rc;
+        note_exec(plan);
         if (int rc = batched_run(plan, plan->bcfg[0], plan->bcfg[1])) return rc;
         plan->ran = true;
         plan->col_split = false;
