@@ -260,6 +260,9 @@ struct gen2_dim
     size_t points() const { return (size_t)P * (size_t)Q; }   // scratch points per sequence
 };
 
+// seconds of an exec's phases
+struct phase_times { double total = 0.0, first = 0.0, second = 0.0, split_a = 0.0, split_b = 0.0; };
+
 struct hpxfft_plan_s
 {
     // problem
@@ -320,11 +323,10 @@ struct hpxfft_plan_s
     bool own_ends = true;        // false: the exec is the middle of a longer one, which stamps start and end itself
     double clock_hz = 1e8;
     bool ran = false;
-    // the host entry point reads its run's times once, when it has waited for it
-    // anyway (three reads by get_measurement: 30 us); not on a plan with captured
-    // execs, whose replays stamp newer ones unseen
-    bool captured = false, host_times_ok = false;
-    double host_times[5] = {};
+    // the last exec's times, once read: one read (8 us) serves all keys.  Not kept
+    // on a plan with captured execs, whose replays stamp newer ones unseen
+    bool captured = false, times_ok = false;
+    phase_times times{};
     bool col_split = false;      // the last run's column pass was a four-step
     bool col_first = false;      // the last run was backward: the column pass before the rows
     double h2d = 0.0, d2h = 0.0;
@@ -950,6 +952,7 @@ constexpr int STAMP_POOL = 64;
 struct stamp_sets
 {
     std::vector<unsigned long long *> free, worn;   // worn: stamped by graphs, oldest first
+    unsigned long long *host = nullptr;              // pinned words that read_times copies a set to
 };
 std::mutex g_stamp_mu;
 std::map<int, stamp_sets> g_stamps;
@@ -970,6 +973,8 @@ struct relaxed_capture
 int grow_stamps(stamp_sets &d)
 {
     relaxed_capture relaxed;
+    if (!d.host) HIPCHK(hipHostMalloc(reinterpret_cast<void **>(&d.host),
+                                       sizeof(unsigned long long) * ST_WORDS, hipHostMallocDefault));
     const size_t bytes = sizeof(unsigned long long) * ST_WORDS * STAMP_POOL;
     unsigned long long *block = nullptr;
     hipStream_t s = nullptr;
@@ -1022,29 +1027,37 @@ int alloc_events(hpxfft_plan_s *p)
     return HPXFFT_OK;
 }
 
-// at the start of an exec (the null stream cannot be captured)
-void note_exec(hpxfft_plan_s *p)
+bool capturing(const hpxfft_plan_s *p)   // (the null stream cannot be captured)
 {
-    p->host_times_ok = false;
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (p->stream && hipStreamIsCapturing(p->stream, &st) == hipSuccess && st != hipStreamCaptureStatusNone)
-        p->captured = true;
+    return p->stream && hipStreamIsCapturing(p->stream, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
 }
 
-// seconds of the last exec's phases, once it has finished
-struct phase_times { double total, first, second, split_a, split_b; };
+// at the start of an exec
+void note_exec(hpxfft_plan_s *p)
+{
+    p->times_ok = false;
+    if (capturing(p)) p->captured = true;
+}
+
+// the last exec's phases, once it has finished.  Waits for the plan's stream: an
+// event of each exec, to wait for no more than that, made two launches of 3 us
+// 9.0 instead of 5.8.  A stream that is being captured is left alone (the copy
+// would become part of the graph).
 int read_times(hpxfft_plan_s *p, phase_times &t)
 {
-    if (p->host_times_ok)
+    if (p->times_ok)
     {
-        const double *h = p->host_times;
-        t = {h[0], h[1], h[2], h[3], h[4]};
+        t = p->times;
         return HPXFFT_OK;
     }
-    std::vector<unsigned long long> w(ST_WORDS);
-    HIPCHK(hipMemcpyAsync(w.data(), p->stamps, sizeof(w[0]) * ST_WORDS, hipMemcpyDeviceToHost, p->stream));
+    if (capturing(p)) return fail(HPXFFT_HIP_ERROR, "phase times: the plan's stream is being captured");
     HIPCHK(hipStreamSynchronize(p->stream));
-    const unsigned long long end = *std::max_element(w.begin() + ST_END, w.end());
+    std::lock_guard<std::mutex> lk(g_stamp_mu);
+    unsigned long long *w = g_stamps[p->device].host;
+    HIPCHK(hipMemcpyAsync(w, p->stamps, sizeof(w[0]) * ST_WORDS, hipMemcpyDeviceToHost, p->stream));
+    HIPCHK(hipStreamSynchronize(p->stream));
+    const unsigned long long end = *std::max_element(w + ST_END, w + ST_WORDS);
     auto s = [&](unsigned long long a, unsigned long long b) { return b > a ? (double)(b - a) / p->clock_hz : 0.0; };
     t.total = s(w[ST_START], end);
     t.first = s(w[ST_START], w[ST_MID]);
@@ -1052,6 +1065,8 @@ int read_times(hpxfft_plan_s *p, phase_times &t)
     // the split lies in the column pass: second after forward execs, first after backward ones
     t.split_a = p->col_first ? s(w[ST_START], w[ST_SPLIT]) : s(w[ST_MID], w[ST_SPLIT]);
     t.split_b = p->col_first ? s(w[ST_SPLIT], w[ST_MID]) : s(w[ST_SPLIT], end);
+    p->times = t;
+    p->times_ok = !p->captured;
     return HPXFFT_OK;
 }
 
@@ -2514,14 +2529,6 @@ int hpxfft_exec_r2c_2d_host(hpxfft_plan plan, double *inout)
         HIPCHK(hipEventSynchronize(e1.ev));
         plan->h2d = elapsed(e0.ev, in_done.ev);
         plan->d2h = elapsed(out_start.ev, e1.ev);
-        if (!plan->captured)
-        {
-            phase_times t{};
-            if (int rc = read_times(plan, t)) return rc;
-            const double h[5] = {t.total, t.first, t.second, t.split_a, t.split_b};
-            std::copy(h, h + 5, plan->host_times);
-            plan->host_times_ok = true;
-        }
         return HPXFFT_OK;
     });
 }

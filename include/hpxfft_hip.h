@@ -175,8 +175,12 @@ int hpxfft_exec_c2r_2d(hpxfft_plan plan, const void *d_spec, void *d_real);
  * pass first: for them "first_fftw" is the column pass and "second_fftw"
  * the row pass; batched plans give their row and column launches.  Unknown keys
  * give 0.0, as std::map::operator[] does in the reference.  The times are
- * stamped by the launches themselves with the device's wall clock (10 ns); a
- * replayed graph stamps them too.  Waits for the plan's stream. */
+ * stamped by the launches themselves with the device's wall clock (10 ns),
+ * the end when the last workgroups have issued their stores; a replayed graph
+ * stamps them too.  The first key asked for after an exec waits for the plan's
+ * stream (while that is being captured: HPXFFT_HIP_ERROR, and the capture goes
+ * on); the others come from the same read, except on a plan with captured
+ * execs, which reads the stamps each time. */
 int hpxfft_get_measurement(hpxfft_plan plan, const char *key, double *value);
 
 /* Replaces hpxfft::shared::loop::write_plans_to_file (loop.cpp:194-212):
