@@ -18,6 +18,17 @@ using hpxfft_dev::RowArgs;
 HPXFFT_DECL_BLUE(f64)
 HPXFFT_DECL_BLUE(f32)
 
+
+// rows or adjacent columns of a workgroup, and its threads
+struct blue_geom { int w, nt; };
+template <typename T, bool COL, int LG = hpxfft_dev::BLUE_MIN_LG> blue_geom blue_shape(int lg)
+{
+    using C = hpxfft_dev::bluecfg<T, LG, COL>;
+    if constexpr (LG < (sizeof(T) == 8 ? hpxfft_dev::BLUE_MAX_LG_F64 : hpxfft_dev::BLUE_MAX_LG_F32))
+        if (lg > LG) return blue_shape<T, COL, LG + 1>(lg);
+    return {C::W, C::NT};
+}
+
 }   // namespace hpxfft_host
 
 #ifdef HPXFFT_INSTANTIATE

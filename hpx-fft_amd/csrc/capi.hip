@@ -779,6 +779,20 @@ std::string gen_method(const hpxfft_dev::GenPlan &g)
            radices(g) + (g.ip ? ", in place: decimation in frequency, then in time)" : ", Stockham)");
 }
 
+// a length that runs in registers (blue_covers), up to the number of its rows or columns
+std::string blue_method(const hpxfft_plan_s *p, const hpxfft_dev::GenPlan &g, bool col)
+{
+    const int lg = ilog2((size_t)g.n);
+    const bool f64 = p->prec == P_F64;
+    const hpxfft_host::blue_geom b =
+        col ? (f64 ? hpxfft_host::blue_shape<double, true>(lg) : hpxfft_host::blue_shape<float, true>(lg))
+            : (f64 ? hpxfft_host::blue_shape<double, false>(lg) : hpxfft_host::blue_shape<float, false>(lg));
+    const int last = 1 << (lg % 4);
+    return "-point Bluestein in registers (two " + std::to_string(g.n) + "-point transforms, radix 16" +
+           (last > 1 ? ", last stage radix " + std::to_string(last) : std::string()) +
+           ", LDS exchange in re/im halves), " + std::to_string(b.nt) + " threads, " + std::to_string(b.w);
+}
+
 int rows_split_width(const hpxfft_plan_s *p, hpxfft_dev::GenPlan &gB);
 
 std::string describe(const hpxfft_plan_s *p)
@@ -791,7 +805,12 @@ std::string describe(const hpxfft_plan_s *p)
         for (int ph = 0; ph < 2; ++ph)
         {
             os << (ph == 0 ? "  row phase" : "  column phase") << ": persistent launch, configuration " << p->bcfg[ph]
-               << " (" << batched_pts(ph, p->bcfg[ph]) << " points per task, " << p->bntasks[ph][p->bcfg[ph]]
+               << " (" << batched_pts(ph, p->bcfg[ph]) << " points per task, "
+               << (ph == 1 && batched_col_width(p->bcfg[1], BATCH_MAX_SIDE) * BATCH_MAX_SIDE > batched_pts(1, p->bcfg[1])
+                       ? std::to_string(batched_col_width(p->bcfg[1], BATCH_MAX_SIDE) * BATCH_MAX_SIDE) +
+                             " on grids of 1024 and 2048 rows, "
+                       : std::string())
+               << p->bntasks[ph][p->bcfg[ph]]
                << " tasks, " << p->bblocks[ph][p->bcfg[ph]] << " workgroups)";
             if (p->effort > 0)
             {
@@ -846,9 +865,11 @@ std::string describe(const hpxfft_plan_s *p)
         else
             os << "    then the r2c split in place (one thread per pair k, Ny/2-k)\n";
     }
+    else if (p->gen_row && blue_covers(p, p->grow))
+        os << "  row r2c kernel (general length): " << p->ny / 2 << blue_method(p, p->grow, false)
+           << " row(s)/workgroup + r2c split; the in-LDS form it replaces: " << gen_method(p->grow) << "\n";
     else if (p->gen_row)
-        os << "  row r2c kernel (general length): " << p->ny / 2 << "-point " << gen_method(p->grow)
-           << (blue_covers(p, p->grow) ? "; forward and inverse transform of each sequence in registers, radix 16" : "") << ", "
+        os << "  row r2c kernel (general length): " << p->ny / 2 << "-point " << gen_method(p->grow) << ", "
            << p->gen_rows << " row(s)/workgroup, "
            << gen_threads(gen_lds_bytes(p, p->grow, (size_t)p->gen_rows * p->grow.n, (size_t)p->gen_rows), p->grow)
            << " threads + r2c split\n";
@@ -874,9 +895,11 @@ std::string describe(const hpxfft_plan_s *p)
         os << "  general column pass autotuned (ms): one level " << p->gcol_ms[0] << ", two levels " << p->gcol_ms[1]
            << "\n";
     if (p->g2c.on) two_level("column c2c", p->g2c);
+    else if (p->gen_col && blue_covers(p, p->gcol))
+        os << "  column c2c kernel (general length): " << p->nx << blue_method(p, p->gcol, true)
+           << " adjacent columns/workgroup; the in-LDS form it replaces: " << gen_method(p->gcol) << "\n";
     else if (p->gen_col)
-        os << "  column c2c kernel (general length): " << p->nx << "-point " << gen_method(p->gcol)
-           << (blue_covers(p, p->gcol) ? "; forward and inverse transform of each sequence in registers, radix 16" : "") << ", "
+        os << "  column c2c kernel (general length): " << p->nx << "-point " << gen_method(p->gcol) << ", "
            << p->gen_w << " adjacent columns/workgroup\n";
     else if (!p->four_step)
     {

@@ -11,8 +11,8 @@
 // registers (16 NB points per thread), with the radix-16 stages and the split
 // exchanges of the long columns (fft_col_long.hpp).  The outputs of the last
 // stage of DFT_L are, thread by thread, the inputs of the next transform's first
-// stage, so the product with Bh takes no exchange: 4 exchanges in all for 4096
-// points (6 where L is no power of 16).  len <= L/2, so the first stage's upper
+// stage, so the product with Bh takes no exchange: 2 exchanges in all for 2^8
+// points, 4 for 2^9 .. 2^12, 6 for 2^13 and 2^14.  len <= L/2, so the first stage's upper
 // inputs are zero, and its upper outputs are never formed.
 // In-LDS form -> this one (us, whole transform): FP64 2039 x 4078 206 -> 106, 1021 x
 // 1024 48 -> 28, 1024 x 8186 168 -> 95, 67 x 1024 30 -> 14; FP32 2039 x 1024 58 -> 34,
