@@ -65,17 +65,23 @@ inline bool col_long_covers(int prec, int lg)
 inline int col_long_width(int prec, int lg, int nt) { return (nt * (prec == P_F64 ? 16 : 32)) >> lg; }
 // threads per workgroup.  2^11 rows: 512 (64-byte row segments, two workgroups
 // per CU; 1024 threads with 128-byte segments were slower up to 4096 reals per
-// row and even beyond).  2^12 rows: 1024 (64-byte segments, one workgroup per
-// CU), except where that leaves CUs idle and the narrow form's twice as many
-// workgroups win: a launch of less than about a third of the 256 CUs (FP64 4096
-// x 512, 65 strips: 23.2 -> 19.5 us; 4096 x 1024, 129 strips: 25.2 against
-// 27.9), or one whose second round would hold a few strips (4096 x 2048, 257
-// strips: 46.3 -> 41.2)
+// row and even beyond).  2^12 rows: 1024 (64-byte segments, one workgroup per CU),
+// except in one or two rounds over the CUs of which the last is at most half full:
+// there the narrow form, with half the columns and twice the workgroups, has one of
+// them per CU where the wide one leaves CUs idle.  Column pass at that many wide
+// strips, wide against narrow (us):
+//   strips      65         113        129        257        321        385        512
+//   FP64    14.4 12.1  15.1 14.1  16.7 20.3  45.8 44.2  35.8 33.4  38.7 42.5  44.6 51.7
+//   FP32    17.8 13.8  18.1 15.9  19.3 24.2  53.0 46.2  42.4 37.9  45.0 47.2  56.4 67.9
+// In a third round it depends on more than the fill (513 strips: FP64 4096 x 4102 57.6
+// against 54.5, 4096 x 4096 72.5 against 78.5; 577: FP32 77.0 against 82.3), and from
+// four on the wide form wins (1025: FP64 101 against 119), so those stay wide.
 inline int col_long_threads(int prec, int lg, size_t ncols, size_t batch)
 {
+    constexpr size_t CUS = 256;   // MI355X
     if (lg == 11) return 512;
     const size_t w = (size_t)col_long_width(prec, lg, 1024), strips = (ncols + w - 1) / w * batch;
-    return strips <= 96 || (strips > 256 && strips <= 288) ? 512 : 1024;
+    return strips <= 2 * CUS && (strips - 1) % CUS < CUS / 2 ? 512 : 1024;
 }
 
 // rows of 2^13 / 2^14 complex points with lane-pair radix-32 stages
