@@ -19,11 +19,11 @@ called directly and through torch.fft.rfft2, on the same transforms beside
 this build's plans; cpu_library times scipy.fft.rfft2 on the host cores beside
 the oracle's CPU port (cpu_baseline).
 
-Every leg reports its launches (event-timed seconds, algorithmic bytes and,
+Every leg reports its launches (stamped seconds, algorithmic bytes and,
 where a committed counter summary covers the workload, HBM traffic) and a
 roofline entry for its longest launch.
 
-roofline: the dominant kernel, the pass with the longest event-timed
+roofline: the dominant kernel, the pass with the longest stamped
 duration on the plan's stream (a four-step column pass is one kernel in two
 launches, phases A and B); achieved = its algorithmic bytes per launch / its
 average launch duration; traffic = its HBM bytes per launch from
@@ -92,7 +92,7 @@ def time_gpu(nx: int, ny: int, precision: str, steps: int, warmup: int, seed: in
     torch.cuda.synchronize()
     wall = time.perf_counter() - t0
     ms = e0.elapsed_time(e1) / steps
-    # per-phase times from the plan's own HIP events (row pass, column pass)
+    # per-phase times from the launches' own stamps (row pass, column pass)
     med = phase_medians(plan, lambda: plan.exec(x.data_ptr(), out.data_ptr()), max(3, min(steps, 10)))
     desc = plan.describe()
     plan_s = plan.measurement("plan")
@@ -103,7 +103,7 @@ def time_gpu(nx: int, ny: int, precision: str, steps: int, warmup: int, seed: in
 
 
 def launches(nx: int, ny: int, s: int, r: dict) -> dict:
-    """Per-launch algorithmic bytes and event-timed duration.  A four-step
+    """Per-launch algorithmic bytes and stamped duration.  A four-step
     column pass is two launches; each is credited half of the column pass's
     2H (phase A reads the spectrum, phase B writes it; the scratch between
     them is not algorithmic)."""
@@ -129,7 +129,7 @@ def measured_traffic(workload: str) -> dict:
 
 
 def phase_medians(plan, run, reps: int = 5) -> dict:
-    """Median event-timed seconds of each phase key over `reps` runs of `run()`
+    """Median stamped seconds of each phase key over `reps` runs of `run()`
     (one exec of `plan` on the plan's stream)."""
     keys = ("first_fftw", "second_fftw", "column_a", "column_b")
     ph = {k: [] for k in keys}
@@ -164,7 +164,7 @@ def launch_table(launches: dict, workload: str) -> dict:
 
 
 def leg_roofline(launches: dict, workload: str) -> dict:
-    """Roofline entry of a leg's dominant launch (the longest event-timed one):
+    """Roofline entry of a leg's dominant launch (the longest stamped one):
     its algorithmic bytes / its duration against the HBM peak, and its HBM
     traffic from the committed counter summary when one covers the workload."""
     name = max(launches, key=lambda k: launches[k][1])
@@ -641,7 +641,7 @@ def main() -> int:
     progress(f"f64 {nx}x{ny}: {r64['ms_per_step']:.4f} ms/step")
     b64 = alg_bytes(nx, ny, 8)
     gbs = b64["total"] / (r64["ms_per_step"] * 1e-3) / 1e9
-    # dominant kernel: the pass with the longest event-timed duration on the
+    # dominant kernel: the pass with the longest stamped duration on the
     # plan's stream.  A four-step column pass is one kernel (tile_kernel) in
     # two launches, phases A and B, credited H each: per launch, its
     # algorithmic bytes, duration and traffic are the two launches' means.

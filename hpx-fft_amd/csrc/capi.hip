@@ -5,7 +5,7 @@
 // (core/src/shared/loop.cpp:158-189): dimensions, the chosen 1-D kernels
 // (instead of FFTW plans), device scratch (instead of the transpose buffer
 // trans_values_vec_, which the fused column pass does not need at full
-// size), twiddle tables, timing events and the measurement map.
+// size), twiddle tables, stamped phase times and the measurement map.
 #include "launch.hpp"
 #include "fft_general.hpp"
 #include "batched.hpp"
