@@ -66,22 +66,25 @@ inline int col_long_width(int prec, int lg, int nt) { return (nt * (prec == P_F6
 // threads per workgroup.  2^11 rows: 512 (64-byte row segments, two workgroups
 // per CU; 1024 threads with 128-byte segments were slower up to 4096 reals per
 // row and even beyond).  2^12 rows: 1024 (64-byte segments, one workgroup per CU),
-// except in one or two rounds over the CUs of which the last is at most half full:
-// there the narrow form, with half the columns and twice the workgroups, has one of
-// them per CU where the wide one leaves CUs idle.  Column pass at that many wide
-// strips, wide against narrow (us):
-//   strips      65         113        129        257        321        385        512
-//   FP64    14.4 12.1  15.1 14.1  16.7 20.3  45.8 44.2  35.8 33.4  38.7 42.5  44.6 51.7
-//   FP32    17.8 13.8  18.1 15.9  19.3 24.2  53.0 46.2  42.4 37.9  45.0 47.2  56.4 67.9
-// In a third round it depends on more than the fill (513 strips: FP64 4096 x 4102 57.6
-// against 54.5, 4096 x 4096 72.5 against 78.5; 577: FP32 77.0 against 82.3), and from
-// four on the wide form wins (1025: FP64 101 against 119), so those stay wide.
+// except where the last of one or two rounds over the CUs is at most half full: there
+// the narrow form, with half the columns and twice the workgroups, has one of them per
+// CU where the wide one leaves CUs idle.  In a second round its 32-byte segments have
+// to be made up for: FP64 gains only while that round is an eighth full; FP32, whose
+// wide kernel spills 32 bytes per lane, as long as in the first.  Whole transforms out
+// of place, buffers beyond the caches, narrow against wide (us, forward / c2r):
+//   strips   64            112           128           136           272           304           384           400
+//   FP64  -4.0 -5.7     -3.4 -5.4     -1.0 -4.0     +2.6 +1.2     -2.8 +0.2     -1.3 +2.7     +1.3 +3.5     +9.6 +13.9
+//   FP32  -4.8 -7.8     -4.0 -7.6     -3.2 -6.9     +3.7 -2.6     -6.2 -4.8     -5.8 -2.7     -4.1 -4.2     +3.4 +8.0
+// (FP64 4096 x 1000, 126 strips, 41.7 -> 38.7; FP32 4096 x 4800, 301, 122.6 -> 118.7.)
+// In a third round it depends on more than the fill (513 strips: FP64 +9.2 +5.5, FP32
+// -4.2 -1.1), and from four on the wide form wins (1025: FP64 columns 101 against 119).
 inline int col_long_threads(int prec, int lg, size_t ncols, size_t batch)
 {
     constexpr size_t CUS = 256;   // MI355X
     if (lg == 11) return 512;
     const size_t w = (size_t)col_long_width(prec, lg, 1024), strips = (ncols + w - 1) / w * batch;
-    return strips <= 2 * CUS && (strips - 1) % CUS < CUS / 2 ? 512 : 1024;
+    const size_t second = prec == P_F64 ? CUS / 8 : CUS / 2;
+    return strips <= CUS / 2 || (strips > CUS && strips <= CUS + second) ? 512 : 1024;
 }
 
 // rows of 2^13 / 2^14 complex points with lane-pair radix-32 stages

@@ -1,8 +1,8 @@
 """The width of one-launch columns of 4096 rows: 512 threads with half the columns where
-the wide form's last round over the 256 CUs, the first or second, is at most half full.
-Numbers of wide strips (4 FP64 or 8 FP32 columns) on both sides of each edge: the plan
-text, and the transform against the oracle (FP64 <= 1e-12, FP32 <= 1e-5, the bounds of
-the other parity tests)."""
+the wide form's last round over the 256 CUs is the first and at most half full, or the
+second and at most an eighth (FP64) or half (FP32) full.  Numbers of wide strips (4 FP64
+or 8 FP32 columns) on both sides of each edge: the plan text, and the transform against
+the oracle (FP64 <= 1e-12, FP32 <= 1e-5, the bounds of the other parity tests)."""
 import numpy as np
 import pytest
 
@@ -10,11 +10,12 @@ import oracle
 
 pytestmark = pytest.mark.gpu
 
-EDGES = [(1, 512), (128, 512), (129, 1024), (256, 1024), (257, 512), (384, 512), (385, 1024), (513, 1024)]
+EDGES = [(1, 512), (128, 512), (129, 1024), (256, 1024), (257, 512), (513, 1024)]
+CASES = [(s, t, p) for s, t in EDGES for p in ("f64", "f32")] + [
+    (288, 512, "f64"), (289, 1024, "f64"), (384, 512, "f32"), (385, 1024, "f32")]
 
 
-@pytest.mark.parametrize("prec", ["f64", "f32"])
-@pytest.mark.parametrize("strips,threads", EDGES)
+@pytest.mark.parametrize("strips,threads,prec", CASES)
 def test_width(gpu, strips, threads, prec):
     import torch
     import hpxfft_amd
@@ -35,7 +36,7 @@ def test_width(gpu, strips, threads, prec):
     assert err <= (1e-12 if prec == "f64" else 1e-5), err
 
 
-@pytest.mark.parametrize("strips,batch,threads", [(32, 4, 512), (43, 3, 1024), (128, 3, 512), (77, 5, 1024)])
+@pytest.mark.parametrize("strips,batch,threads", [(32, 4, 512), (43, 3, 1024), (96, 3, 512), (97, 3, 1024)])
 def test_width_counts_the_batch(gpu, strips, batch, threads):
     import hpxfft_amd
     p = hpxfft_amd.Plan(4096, 2 * (strips * 4 - 1), batch=batch, precision="f64")
